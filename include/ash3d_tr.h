@@ -217,7 +217,8 @@ enum {
   ASH3D_TUNE_PART_SHAPE_X = 9, /* tile shape of the partitioned solves (0 or 1; defaults 1, 1, 0), x lines */
   ASH3D_TUNE_PART_SHAPE_Y = 10,
   ASH3D_TUNE_PART_SHAPE_Z = 11,
-  /* streamed y/z advection: 0 cuts the lines of a workgroup into segments;
+  /* streamed y/z advection (in-place sweeps along more than 64 cells; the
+   * others run in register tiles, which take no setting): 0 cuts the lines of a workgroup into segments;
    * 1..4 gives each wave of a workgroup one bin group of the same whole
    * lines, so the per-cell fields are read once for all of them */
   ASH3D_TUNE_ADV_GROUPS_Y = 12,
@@ -241,8 +242,8 @@ enum {
    * ensemble steps): 1 the second horizontal sweep and the vertical sweep
    * in one pass (the first sweep writes the ts1 slot, the fused pass reads
    * it with the halo along its lines and writes ts0; bitwise the split
-   * sweeps), 0 three separate in-place sweeps; default 1 on grids of at
-   * least 2^24 interior cells, 0 below */
+   * sweeps), 0 three separate sweeps; default 1 on grids of at least 2^24
+   * interior cells with more than 10 bins, 0 otherwise */
   ASH3D_TUNE_ADV_FUSED = 17,
   /* partitioned mode, eager steps: the most Jacobi sweeps a line may take
    * (0..12; 0 never; default 12).  y and z theta-scheme sweeps whose lines

@@ -357,6 +357,10 @@ static hipError_t advect_any(hipStream_t s, const AdvArgs &a, int nb, LaunchSpec
     hipError_t e = sp ? spec_advect_x_rows(a, sp) : launch_advect_x_rows(s, a);
     if (e != hipErrorInvalidValue) return e;
     (void)hipGetLastError();  // row too long for one workgroup: stream it
+  } else {
+    hipError_t e = advect_tile(s, a, sp);
+    if (e != hipErrorInvalidValue) return e;
+    (void)hipGetLastError();  // no tiles for this sweep: stream it
   }
   switch (nb) {
     case 1: return launch_nb<1>(s, a, sp);

@@ -441,6 +441,43 @@ int sweep_advect(ash3d_tr_ctx *x, int dir, double dt, const int32_t *is_aloft, c
   return 0;
 }
 
+// The advection sweeps of a step through the ts1 slot: y from ts0 into ts1
+// and z from ts1 into ts0 in register tiles, x in place on the slot that
+// holds the state by then.  Full passes of Set_BC(1) between the sweeps
+// would leave what is read as it is: along y and z the ghosts are zeros
+// (read as such), along x zeros or, with periodic x, the copies written
+// here before the x sweep.  Not for a periodic step without diffusion,
+// whose x ghosts in ts0 stay observable.
+bool advect_through_ts1(const ash3d_tr_ctx *x, const int32_t *bounds, bool zg) {
+  return (zg || !x->periodic) && advect_tile_applies(make_line_geom(x->d, 1, bounds), false) &&
+         advect_tile_applies(make_line_geom(x->d, 2, bounds), false);
+}
+AdvArgs through_ts1_args(ash3d_tr_ctx *x, int dir, double dt, const int32_t *is_aloft, const int32_t *bounds,
+                         bool x_first) {
+  AdvArgs a = advect_args(x, dir, dt, is_aloft, bounds, dir == 1 || (dir == 0 && x_first) ? x->ts0() : x->ts1());
+  a.zg = (x->periodic && dir == 0) ? 0 : 1;
+  if (dir == 1) a.cout = x->ts1();
+  if (dir == 2) a.cout = x->ts0();
+  return a;
+}
+int step_advect_ts1(ash3d_tr_ctx *x, int first, double dt, const int32_t *is_aloft, const int32_t *bounds) {
+  int rc = check_bounds(x, bounds);
+  if (rc) return rc;
+  if (!(dt >= 0.0)) return fail(ASH3D_TR_EINVAL, "dt must be >= 0 (got %g)", dt);
+  const int order[3] = {first, 1 - first, 2};
+  for (int dir : order) {
+    const AdvArgs a = through_ts1_args(x, dir, dt, is_aloft, bounds, first == 0);
+    if (dir == 0 && x->periodic) {
+      ProfScope ps(x, ASH3D_PROF_BC);
+      HIPCHK(launch_set_bc2_face(x->stream, x->d, 1, 0, a.c0));
+    }
+    ProfScope ps(x, ASH3D_PROF_ADVECT_X + dir);
+    HIPCHK(launch_advect(x->stream, a, x->nb_adv[dir]));
+  }
+  x->ts1_state = TS1_MIRROR;
+  return 0;
+}
+
 // Transposed kappa, sigma_nx and kx for the x-line solves.
 int ensure_tgeom(ash3d_tr_ctx *x) {
   int rc = 0;
@@ -924,10 +961,11 @@ int ash3d_tr_create(const ash3d_tr_desc *desc, ash3d_tr_ctx **out) {
   x->device = desc->device;
   x->host = *desc;
   x->d = make_dims(desc->nx, desc->ny, desc->nz, desc->ns);
-  // the fused advection pass pays off on large grids (measured: 9 % less
-  // advection time on 1440x720x80, 5 % more on the 120-400 x 80-300 x
-  // 40-60 ensemble grids)
-  x->adv_fused = (long long)desc->nx * desc->ny * desc->nz >= (1LL << 24) ? 1 : 0;
+  // the fused advection pass pays off on large grids with many bins
+  // (advection per step on 1440x720x80, fused against three sweeps: 20 bins
+  // 21.1 against 23.4 ms, 10 bins 12.2 against 12.1, 4 bins 5.71 against
+  // 5.47; on 360x240x50x15 1.33 against 1.01 ms)
+  x->adv_fused = (long long)desc->nx * desc->ny * desc->nz >= (1LL << 24) && desc->ns > 10 ? 1 : 0;
   x->periodic = desc->is_periodic ? 1 : 0;
   x->zscaling = desc->zscaling_id;
   x->limiter = desc->limiter;
@@ -1168,6 +1206,23 @@ int ash3d_tr_advect_horz(ash3d_tr_ctx *x, int32_t itoggle, double dt, const int3
   int32_t b[6];
   full_bounds(x, b);
   const int first = (itoggle % 2 == 0) ? 1 : 0;
+  if (!x->periodic) {
+    // out of place into ts1 and back: y runs in register tiles at any line
+    // length; the second routine's Set_BC(1) would rewrite ghosts that are
+    // zero in ts0 already (and are read as zeros from ts1)
+    if (!(dt >= 0.0)) return fail(ASH3D_TR_EINVAL, "dt must be >= 0 (got %g)", dt);
+    if ((rc = set_bc1(x, true))) return rc;
+    for (int q = 0; q < 2; ++q) {
+      const int dir = q == 0 ? first : 1 - first;
+      AdvArgs a = advect_args(x, dir, dt, is_aloft, b, q == 0 ? x->ts0() : x->ts1());
+      a.cout = q == 0 ? x->ts1() : x->ts0();
+      a.zg = 1;
+      ProfScope ps(x, ASH3D_PROF_ADVECT_X + dir);
+      HIPCHK(launch_advect(x->stream, a, x->nb_adv[dir]));
+    }
+    x->ts1_state = TS1_MIRROR;
+    return 0;
+  }
   if ((rc = sweep_advect(x, first, dt, is_aloft, b, true, true))) return rc;
   return sweep_advect(x, 1 - first, dt, is_aloft, b, true, false);
 }
@@ -1265,6 +1320,8 @@ int ash3d_tr_step(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t use_diffusi
       HIPCHK(launch_advect_hz(x->stream, h, z));
     }
     x->ts1_state = TS1_MIRROR;
+  } else if (advect_through_ts1(x, b, zg)) {
+    if ((rc = step_advect_ts1(x, first, dt, is_aloft, b))) return rc;
   } else {
     for (int q = 0; q < 3; ++q) {
       const int dir = order[q];
@@ -2097,9 +2154,13 @@ int ash3d_tr_step_subgrid(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t use
     for (int q = 0; q < 6; ++q) bounds[q] = b[q];
   const int first = (itime % 2 == 0) ? 1 : 0;
   const bool again = x->periodic != 0;
-  if ((rc = sweep_advect(x, first, dt, is_aloft, b, false, false))) return rc;
-  if ((rc = sweep_advect(x, 1 - first, dt, is_aloft, b, again, false))) return rc;
-  if ((rc = sweep_advect(x, 2, dt, is_aloft, b, again, false))) return rc;
+  if (advect_through_ts1(x, b, use_diffusion != 0)) {
+    if ((rc = step_advect_ts1(x, first, dt, is_aloft, b))) return rc;
+  } else {
+    if ((rc = sweep_advect(x, first, dt, is_aloft, b, false, false))) return rc;
+    if ((rc = sweep_advect(x, 1 - first, dt, is_aloft, b, again, false))) return rc;
+    if ((rc = sweep_advect(x, 2, dt, is_aloft, b, again, false))) return rc;
+  }
   if (use_diffusion) {
     const int dfirst = (itime % 2 == 0) ? 0 : 1;
     {
@@ -2258,13 +2319,12 @@ int ens_member_specs(ash3d_tr_ctx *x, int itime, double dt, double imp_fac, cons
   } else {
     for (int i = 0; i < 3; ++i) {
       const int dir = order[i];
+      const AdvArgs a = through_ts1_args(x, dir, dt, is_aloft, b, first == 0);
       if (dir == 0) {
         // (periodic x: the x ghosts the sweep reads are the periodic copies)
-        if (x->periodic) spec_set_bc2_face(x->d, 1, 0, x->ts0(), &slots[q]);
+        if (x->periodic) spec_set_bc2_face(x->d, 1, 0, a.c0, &slots[q]);
         ++q;
       }
-      AdvArgs a = advect_args(x, dir, dt, is_aloft, b, x->ts0());
-      a.zg = (x->periodic && dir == 0) ? 0 : 1;
       hipError_t e = spec_advect(a, x->nb_adv[dir], &slots[q++]);
       if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "ensemble advection dir %d: %s", dir, hipGetErrorString(e));
     }

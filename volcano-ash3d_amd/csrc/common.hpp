@@ -271,6 +271,10 @@ hipError_t launch_advect_hz(hipStream_t s, const AdvArgs &h, const AdvArgs &z);
 // out[c] = dt / kap[c] for the n cells (the fused pass's cached dt/kappa)
 hipError_t launch_cell_dtv(hipStream_t s, const double *kap, double *out, long long n, double dt);
 hipError_t spec_advect_hz(const AdvArgs &h, const AdvArgs &z, LaunchSpec *sp);
+// y and z sweeps in register tiles (advect_tile.hip): issue the launch, or
+// describe it in sp; hipErrorInvalidValue where advect_tile_applies is false
+hipError_t advect_tile(hipStream_t s, const AdvArgs &a, LaunchSpec *sp);
+bool advect_tile_applies(const LineGeom &g, bool in_place);
 hipError_t launch_advect_x_rows(hipStream_t s, const AdvArgs &a);
 // the launch launch_advect_x_rows would issue (hipErrorInvalidValue: the
 // row needs the streamed kernel)

@@ -40,4 +40,18 @@ __device__ inline double limited_flux(int lim, double dqm, double dq0, double dq
   return 0.5 * aus * (1.0 - dtv * aus) * ldq;
 }
 
+// limited_flux without branches (every selection a select), so that the
+// divisions of a tile's interfaces overlap instead of running one behind
+// the other: the same bits.  LIM: the limiter, or -1 to read it from lim.
+template <int LIM>
+__device__ inline double limited_flux_flat(int lim, double dqm, double dq0, double dqp, double u, double dtv) {
+  const double dqu = (u > 0.0) ? dqm : dqp;
+  const double quot = dqu / dq0;
+  const double theta = fabs(dqu) > 3.0 * fabs(dq0) ? copysign(3.0, dqu * dq0) : quot;
+  const double ldq = limited_dq(LIM < 0 ? lim : LIM, dq0, dqu, theta);
+  const double aus = fabs(u);
+  const double f = 0.5 * aus * (1.0 - dtv * aus) * ldq;
+  return fabs(dq0) <= EPS_THRESH ? 0.0 : f;
+}
+
 }  // namespace ash3d
