@@ -769,24 +769,6 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
     x->ts1_state = TS1_MIRROR;
     return 0;
   }
-  const bool transposed = (dir == 0);
-  if (transposed) {
-    // explicit x lines as the y lines of the transposed grid (x and y swapped)
-    const Dims &d = x->d;
-    if ((rc = ensure_tgeom(x))) return rc;
-    if (!x->tq && (rc = dev_alloc(&x->tq, x->n_conc()))) return rc;
-    {
-      ProfScope ps(x, ASH3D_PROF_TRANSPOSE);
-      HIPCHK(launch_transpose_xy(x->stream, x->ts0(), x->tq, d.nx + 4, d.ny + 4, (long long)(d.nz + 4) * d.ns));
-    }
-    const int32_t tb[6] = {bounds[2], bounds[3], bounds[0], bounds[1], bounds[4], bounds[5]};
-    a.d = make_dims(d.ny, d.nx, d.nz, d.ns);
-    a.g = make_line_geom(a.d, 1, tb);
-    a.c0 = x->tq;
-    a.kap = x->tkap;
-    a.sig = x->tsx;
-    a.kk = x->tkx;
-  }
   if (use_cn) {
     if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a))) return rc;
     ProfScope ps(x, ASH3D_PROF_DIFFUSE_X + dir);  // one record for both kernels
@@ -798,12 +780,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
     else if (tp != 2) HIPCHK(launch_diff_cn(x->stream, a, x->nb_diff[dir]));
   } else {
     ProfScope ps(x, ASH3D_PROF_DIFFUSE_X + dir);
-    HIPCHK(launch_diff_explicit(x->stream, a, x->nb_diff[dir]));
-  }
-  if (transposed) {
-    ProfScope ps(x, ASH3D_PROF_TRANSPOSE);
-    HIPCHK(launch_transpose_xy(x->stream, x->tq, x->ts0(), x->d.ny + 4, x->d.nx + 4,
-                               (long long)(x->d.nz + 4) * x->d.ns));
+    HIPCHK(launch_diff_explicit(x->stream, a, x->periodic));
   }
   x->ts1_state = TS1_MIRROR;
   return 0;
@@ -1945,7 +1922,7 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
   if (x->prof_on) return fail(ASH3D_TR_EINVAL, "kernel timing is on; switch it off before capturing");
   if (use_diffusion && use_cn && !(x->lu[0] && x->lu[1] && x->lu[2] && x->junk))
     return fail(ASH3D_TR_EINVAL, "capture after an eager step (line-solve factors not allocated)");
-  if (use_diffusion && !x->tgeom_valid)
+  if (use_diffusion && use_cn && !x->tgeom_valid)
     return fail(ASH3D_TR_EINVAL, "capture after an eager step (transposed geometry not built)");
   HIPCHK(hipStreamSynchronize(x->stream));
   const int slot = itime % 2;
@@ -1975,7 +1952,7 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     x->graph_lu_on[slot][k] = x->lu_args_set[k];
     x->graph_lu[slot][k] = x->lu_args[k];
   }
-  x->graph_tgeom[slot] = use_diffusion != 0;
+  x->graph_tgeom[slot] = use_diffusion && use_cn;
   return 0;
 }
 

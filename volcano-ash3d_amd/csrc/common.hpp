@@ -279,7 +279,9 @@ hipError_t launch_advect_x_rows(hipStream_t s, const AdvArgs &a);
 // the launch launch_advect_x_rows would issue (hipErrorInvalidValue: the
 // row needs the streamed kernel)
 hipError_t spec_advect_x_rows(const AdvArgs &a, LaunchSpec *sp);
-hipError_t launch_diff_explicit(hipStream_t s, const DiffArgs &a, int nb);
+// explicit sweep of a in place (x lines too in the state's own layout); the
+// ts1 slot a.scratch_b is scratch
+hipError_t launch_diff_explicit(hipStream_t s, const DiffArgs &a, int periodic);
 hipError_t launch_diff_cn(hipStream_t s, const DiffArgs &a, int nb);
 // the row factors L, R of every cell of the sweep's lines (bin-independent)
 hipError_t launch_line_lr(hipStream_t s, const DiffArgs &a, double *lr);

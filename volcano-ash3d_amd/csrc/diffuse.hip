@@ -1,5 +1,5 @@
-// Diffusion sweeps: explicit diff_{x,y,z} (src/Diffusion.F90:266-650) and
-// the theta-scheme diffCN_{x,y,z} (src/Diffusion.F90:671-1428) with the
+// Diffusion sweeps: the theta-scheme diffCN_{x,y,z} (src/Diffusion.F90:
+// 671-1428; the explicit ones are in diffuse_explicit.hip) with the
 // tridiagonal solve of LAPACK dgtsv (Gaussian elimination with partial
 // pivoting), which the reference calls once per line and bin.
 //
@@ -186,89 +186,6 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
 
 __global__ void k_zero_i32(int *p) { *p = 0; }
 __global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
-
-template <int DIR, int NB>
-__global__ __launch_bounds__(kBlock) void k_diff_explicit(DiffArgs A) {
-  const Dims d = A.d;
-  const LineGeom g = A.g;
-  const TileGroup tg = xcd_tile_group(blockIdx.x, (d.ns + NB - 1) / NB);
-  const long long gid = tg.tile * kBlock + threadIdx.x;
-  if (gid >= (long long)g.Na * g.Nb) return;
-  const int a = (int)(gid % g.Na) + 1;
-  const int b = (int)(gid / g.Na) + 1;
-  const int n0 = tg.group * NB;
-  const int N = g.N, rmin = g.rmin, rmax = g.rmax;
-  const long long sL = line_stride(d, DIR), base = line_base(d, DIR, a, b);
-  const long long kS = kline_stride(d, DIR), kB = kline_base(d, DIR, a, b);
-  const bool line_on = a >= g.a0 && a <= g.a1 && b >= g.b0 && b <= g.b1;
-  double *c = A.c0;
-  bool exists[NB], on[NB];
-  bool any_on = false;
-#pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    exists[u] = (n0 + u) < d.ns;
-    on[u] = exists[u] && line_on && A.aloft.on(n0 + u);
-    any_on = any_on || on[u];
-  }
-  if (any_on) {
-    const double dt = A.dt;
-    // window: q_{r-1}, kap_{r-1}, K_{r-1}; interface r-1 quantities
-    double qm[NB], dqm[NB];
-#pragma unroll
-    for (int u = 0; u < NB; ++u) qm[u] = dqm[u] = 0.0;
-    double kapm = 1.0, Km = 0.0, sigm = 0.0, Am = 0.0;
-    for (int r = rmin - 1; r <= rmax + 1; ++r) {
-      const long long cell = base + sL * (long long)(r + 1);
-      const double kap0 = A.kap[cell];
-      const double K0 = A.kk[kB + kS * (long long)r];
-      double q0[NB];
-#pragma unroll
-      for (int u = 0; u < NB; ++u) q0[u] = exists[u] ? c[cell + d.ncell * (long long)(n0 + u)] : 0.0;
-      if (r >= rmin) {
-        // interface I = r (:357-359)
-        const double sig0 = A.sig[cell];
-        const double ds = 2.0 * sig0 / (kapm + kap0);
-        const double kds = 0.5 * (Km + K0) * ds;
-        const double A0 = dt * kds;
-        const int cc = r - 1;
-        if (cc >= rmin) {
-          // cell cc = r-1 (:367-372): interfaces cc (=r-1) and cc+1 (=r)
-          const double sR = sig0 / kapm;  // sig_{c+1}/kap_c
-          const double sLf = sigm / kapm; // sig_c/kap_c
-#pragma unroll
-          for (int u = 0; u < NB; ++u) {
-            const double dq0 = q0[u] - qm[u];
-            if (on[u]) {
-              const double LF = A0 * dq0 * sR;
-              const double RF = -(Am * dqm[u] * sLf);
-              c[base + sL * (long long)(cc + 1) + d.ncell * (long long)(n0 + u)] = qm[u] + (LF + RF);
-            }
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) dqm[u] = q0[u] - qm[u];
-        Am = A0;
-        sigm = sig0;
-      }
-#pragma unroll
-      for (int u = 0; u < NB; ++u) qm[u] = q0[u];
-      kapm = kap0;
-      Km = K0;
-    }
-  }
-  // zero fill of ts1 then copy (:314, :385-386)
-#pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    if (!exists[u]) continue;
-    const long long bofs = d.ncell * (long long)(n0 + u);
-    if (!on[u]) {
-      for (int r = 1; r <= N; ++r) c[base + sL * (long long)(r + 1) + bofs] = 0.0;
-    } else {
-      for (int r = 1; r < rmin; ++r) c[base + sL * (long long)(r + 1) + bofs] = 0.0;
-      for (int r = rmax + 1; r <= N; ++r) c[base + sL * (long long)(r + 1) + bofs] = 0.0;
-    }
-  }
-}
 
 // theta-scheme line solve.  Row l (cell c = rmin-1+l) of the system
 // (:807-853):
@@ -1188,21 +1105,6 @@ hipError_t launch_cn_xrows_tx(hipStream_t s, const DiffArgs &a, const XState &x,
   }
 }
 
-template <template <int, int> class K, int NB>
-struct dummy {};
-
-template <int NB>
-hipError_t launch_explicit_nb(hipStream_t s, const DiffArgs &a) {
-  const long long lines = (long long)a.g.Na * a.g.Nb;
-  dim3 grid((unsigned)(padded_tiles((lines + kBlock - 1) / kBlock) * ((a.d.ns + NB - 1) / NB)));
-  switch (a.g.dir) {
-    case 0: hipLaunchKernelGGL((k_diff_explicit<0, NB>), grid, dim3(kBlock), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((k_diff_explicit<1, NB>), grid, dim3(kBlock), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_diff_explicit<2, NB>), grid, dim3(kBlock), 0, s, a); break;
-  }
-  return hipGetLastError();
-}
-
 template <int NB>
 hipError_t launch_cn_nb(hipStream_t s, const DiffArgs &a) {
   const long long lines = (long long)a.g.Na * a.g.Nb;
@@ -1216,15 +1118,6 @@ hipError_t launch_cn_nb(hipStream_t s, const DiffArgs &a) {
 }
 
 }  // namespace
-
-hipError_t launch_diff_explicit(hipStream_t s, const DiffArgs &a, int nb) {
-  switch (nb) {
-    case 1: return launch_explicit_nb<1>(s, a);
-    case 2: return launch_explicit_nb<2>(s, a);
-    case 4: return launch_explicit_nb<4>(s, a);
-    default: return launch_explicit_nb<8>(s, a);
-  }
-}
 
 hipError_t launch_line_lr(hipStream_t s, const DiffArgs &a, double *lr) {
   const long long cells = (long long)a.g.Na * a.g.N * a.g.Nb;
