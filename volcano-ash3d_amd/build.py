@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libash3d_tr.so")
-SOURCES = ["ash3d_tr.hip", "bc.hip", "advect.hip", "advect_tile.hip", "advect_x.hip", "diffuse.hip", "diffuse_explicit.hip", "totals.hip", "transpose.hip",
+SOURCES = ["ash3d_tr.hip", "bc.hip", "advect.hip", "advect_tile.hip", "advect_x.hip", "diffuse.hip", "diffuse_explicit.hip", "cn_exact.hip", "totals.hip", "transpose.hip",
            "adjoint.hip", "meteo.hip", "linesolve.hip", "products.hip", "source.hip", "advect_hz.hip"]
 ARCH = os.environ.get("ASH3D_OFFLOAD_ARCH", "gfx950")
 

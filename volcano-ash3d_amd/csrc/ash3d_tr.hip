@@ -135,7 +135,7 @@ struct ash3d_tr_ctx {
   // needs instead of both with the choice made on the device.  The row
   // ratios and the flagged line count come back with it (njl_h, rho_h,
   // rhoj_h, in the same pinned block).
-  int *ndom_h = nullptr, *njl_h = nullptr;
+  int *ndom_h = nullptr, *njl_h = nullptr;  // ndom_h: two counts per direction (k_line_lu's ndom[0], ndom[1])
   unsigned long long *rho_h = nullptr, *rhoj_h = nullptr;
   hipEvent_t ndom_ev[3] = {};
   int ndom_state[3] = {0, 0, 0};
@@ -578,15 +578,15 @@ int host_ndom(ash3d_tr_ctx *x, int dir) {
         x->ndom_h = nullptr;
         return -1;
       }
-      x->njl_h = x->ndom_h + 4;
-      x->rho_h = (unsigned long long *)(x->ndom_h + 8);
+      x->njl_h = x->ndom_h + 6;
+      x->rho_h = (unsigned long long *)(x->ndom_h + 10);
       x->rhoj_h = x->rho_h + 3;
     }
     if (!x->ndom_ev[dir] && hipEventCreateWithFlags(&x->ndom_ev[dir], hipEventDisableTiming) != hipSuccess) {
       x->ndom_ev[dir] = nullptr;
       return -1;
     }
-    if (hipMemcpyAsync(x->ndom_h + dir, x->lu_ndom[dir], sizeof(int), hipMemcpyDeviceToHost, x->stream) !=
+    if (hipMemcpyAsync(x->ndom_h + 2 * dir, x->lu_ndom[dir], 2 * sizeof(int), hipMemcpyDeviceToHost, x->stream) !=
             hipSuccess ||
         hipMemcpyAsync(x->rho_h + dir, x->lu_rho[dir], sizeof(unsigned long long), hipMemcpyDeviceToHost,
                        x->stream) != hipSuccess ||
@@ -603,8 +603,11 @@ int host_ndom(ash3d_tr_ctx *x, int dir) {
     if (hipEventQuery(x->ndom_ev[dir]) != hipSuccess) return -1;
     x->ndom_state[dir] = 2;
   }
-  return x->ndom_h[dir];
+  return x->ndom_h[2 * dir];
 }
+
+// the same for the count of lines whose elimination interchanges rows
+int host_nswap(ash3d_tr_ctx *x, int dir) { return host_ndom(x, dir) < 0 ? -1 : x->ndom_h[2 * dir + 1]; }
 
 // Jacobi sweeps for a theta-scheme sweep of y or z lines that would
 // otherwise be solved in dgtsv order (partitioned mode, eager steps): the
@@ -693,6 +696,27 @@ int try_cn_partitioned(ash3d_tr_ctx *x, int dir, DiffArgs &a, int *rc, bool adjo
   return hn == 0 ? 2 : 1;
 }
 
+// dgtsv-order solves of a sweep (x lines: a describes the transposed grid):
+// the kernel without row interchanges where no line has any, the general one
+// where some has, and while the host does not know (the first sweep after a
+// factorisation, captures) both, of which the device runs one.  A sweep that
+// the partitioned solves may have taken (a.sel = 2) leaves only its
+// non-dominant case, to the general kernel.
+int solve_dgtsv_order(ash3d_tr_ctx *x, int dir, DiffArgs &a) {
+  if (a.sel != 2) {
+    const int sw = host_nswap(x, dir);
+    if (sw <= 0) {
+      a.sel = 4;
+      HIPCHK(launch_cn_exact(x->stream, a, dir == 0 ? &x->d : nullptr, x->ts0()));
+      if (sw == 0) return 0;
+    }
+    a.sel = sw < 0 ? 3 : 0;
+  }
+  if (dir == 0) HIPCHK(launch_diff_cn_xrows(x->stream, a, x->d, x->ts0(), x->nb_diff[0], x->x_tile));
+  else HIPCHK(launch_diff_cn(x->stream, a, x->nb_diff[dir]));
+  return 0;
+}
+
 // Arguments of a diffusion sweep of direction dir over the state ts0
 DiffArgs diff_args(ash3d_tr_ctx *x, int dir, double dt, double imp_fac, const int32_t *is_aloft,
                    const int32_t *bounds) {
@@ -764,7 +788,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
       const int tp = try_cn_partitioned(x, 0, a, &rc);
       if (rc) return rc;
       if (sw > 0 && tp != 2) return fail(ASH3D_TR_EDEVICE, "x-line Jacobi sweeps without the partitioned solves");
-      if (tp != 2) HIPCHK(launch_diff_cn_xrows(x->stream, a, d, x->ts0(), x->nb_diff[0], x->x_tile));
+      if (tp != 2 && (rc = solve_dgtsv_order(x, 0, a))) return rc;
     }
     x->ts1_state = TS1_MIRROR;
     return 0;
@@ -777,7 +801,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
     const int k = tp == 0 ? jacobi_iters(x, dir) : -1;
     x->jacobi_last[dir] = k + 1;
     if (k >= 0) HIPCHK(launch_diff_cn_jacobi(x->stream, a, x->nb_diff[dir], k));
-    else if (tp != 2) HIPCHK(launch_diff_cn(x->stream, a, x->nb_diff[dir]));
+    else if (tp != 2 && (rc = solve_dgtsv_order(x, dir, a))) return rc;
   } else {
     ProfScope ps(x, ASH3D_PROF_DIFFUSE_X + dir);
     HIPCHK(launch_diff_explicit(x->stream, a, x->periodic));

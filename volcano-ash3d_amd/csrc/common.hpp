@@ -175,9 +175,11 @@ struct DiffArgs {
   const uint8_t *piv;
   const int *sing;
   // number of lines of the sweep whose matrix is not diagonally dominant
-  // (from k_line_lu); sel = 1: the kernel runs only when it is zero (the
-  // partitioned solves), sel = 2: only when it is not (their dgtsv-order
-  // alternative), sel = 0: always
+  // (from k_line_lu) and, in ndom[1], of lines whose elimination interchanges
+  // rows; sel = 1: the partitioned solves run only when ndom[0] is zero,
+  // sel = 2: only when it is not (their dgtsv-order alternative), sel = 3
+  // and 4: the dgtsv-order kernels with, and without, row interchanges only
+  // when ndom[1] is not zero, and zero; sel = 0: always
   const int *ndom;
   int sel;
   double *junk;        // kJunk doubles that masked-off lanes store to
@@ -283,6 +285,10 @@ hipError_t spec_advect_x_rows(const AdvArgs &a, LaunchSpec *sp);
 // ts1 slot a.scratch_b is scratch
 hipError_t launch_diff_explicit(hipStream_t s, const DiffArgs &a, int periodic);
 hipError_t launch_diff_cn(hipStream_t s, const DiffArgs &a, int nb);
+// dgtsv-order solves of a sweep without row interchanges (a.sel = 4: the
+// kernel returns at once when a.ndom[1] is not zero).  x lines: a describes the x<->y
+// transposed grid, orig and c_orig the state; otherwise null
+hipError_t launch_cn_exact(hipStream_t s, const DiffArgs &a, const Dims *orig, double *c_orig);
 // the row factors L, R of every cell of the sweep's lines (bin-independent)
 hipError_t launch_line_lr(hipStream_t s, const DiffArgs &a, double *lr);
 // partitioned line solves (linesolve.hip): offsets of cell r of line (a, b)

@@ -68,6 +68,8 @@ __global__ __launch_bounds__(kBlock) void k_line_lr(DiffArgs A, double *lr) {
 // *ndom counts the lines that are not diagonally dominant M-matrix rows
 // (some L or R negative or not finite, or theta < 0): the partitioned
 // solves, which eliminate without pivoting, are used only when it is zero.
+// ndom[1] counts the lines with an interchange (a row dominant in itself is
+// interchanged when the next row's sub-diagonal entry is larger still).
 template <int DIR>
 __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint8_t *piv, int *sing, int *ndom,
                                                    unsigned long long *rho, uint8_t *jl, unsigned long long *rho_j,
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
   const double *Lf = A.lr, *Rf = A.lr + d.ncell;
   double *fF = lu, *fD = lu + d.ncell, *fDU = fD + d.ncell, *fDL = fDU + d.ncell;
   int singular = 0;
-  bool dom = true;
+  bool dom = true, swaps = false;
   double rho_line = 0.0;  // largest (|DL| + |DU|) / |D| of the line's rows
   double Dc = 0.0, DUc = 0.0;
   // row factors PF rows ahead
@@ -153,6 +155,7 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
         DUc = temp;
         Dc = newDi;
         p_i = 1;
+        swaps = true;
       }
       fF[fo] = fact;
       piv[fo] = p_i;
@@ -167,6 +170,7 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
   fD[base + sL * (long long)(rmin + n)] = Dc;
   sing[gid] = singular;
   if (!dom) atomicAdd(ndom, 1);
+  if (swaps) atomicAdd(ndom + 1, 1);
   // the sweep's largest row ratio (non-negative doubles order as their bit
   // patterns); lines that are not dominant count as 1
   const double r = (dom && rho_line < 1.0) ? rho_line : 1.0;
@@ -184,8 +188,15 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
   }
 }
 
-__global__ void k_zero_i32(int *p) { *p = 0; }
-__global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
+// the counts and ratios that k_line_lu accumulates
+__global__ void k_zero_counts(int *ndom, unsigned long long *rho, unsigned long long *rho_j, int *njl) {
+  ndom[0] = ndom[1] = 0;
+  if (rho) *rho = 0ull;
+  if (rho_j) {
+    *rho_j = 0ull;
+    *njl = 0;
+  }
+}
 
 // theta-scheme line solve.  Row l (cell c = rmin-1+l) of the system
 // (:807-853):
@@ -207,7 +218,7 @@ __global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
 template <int DIR, int NB>
 __global__ __launch_bounds__(kBlock) void k_diff_cn(DiffArgs A) {
   constexpr int PF = 4;  // rows in flight per stream
-  if (A.sel == 2 && *A.ndom == 0) return;  // the partitioned solves ran (uniform)
+  if ((A.sel == 2 && A.ndom[0] == 0) || (A.sel == 3 && A.ndom[1] == 0)) return;  // another kernel ran (uniform)
   const Dims d = A.d;
   const LineGeom g = A.g;
   const TileGroup tg = xcd_tile_group(blockIdx.x, (d.ns + NB - 1) / NB);
@@ -838,7 +849,7 @@ struct XState {
 template <int NB, int TX>
 __global__ __launch_bounds__(64) void k_diff_cn_xrows(DiffArgs A, XState X) {
   constexpr int PF = 4;  // rows in flight; TX cells per LDS tile
-  if (A.sel == 2 && *A.ndom == 0) return;  // the partitioned solves ran (uniform)
+  if ((A.sel == 2 && A.ndom[0] == 0) || (A.sel == 3 && A.ndom[1] == 0)) return;  // another kernel ran (uniform)
   __shared__ double s_t[NB][64][TX + 1];
   __shared__ long long s_row[64];          // original offset of cell -1 of each lane's line (-1: none)
   __shared__ unsigned char s_on[64];       // line_on of each lane
@@ -1135,12 +1146,7 @@ hipError_t launch_line_lu(hipStream_t s, const DiffArgs &a, double *lu, uint8_t 
   if ((jl == nullptr) != (rho_j == nullptr) || (jl == nullptr) != (njl == nullptr)) return hipErrorInvalidValue;
   const long long lines = (long long)a.g.Na * a.g.Nb;
   dim3 grid((unsigned)((lines + kBlock - 1) / kBlock));
-  hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, s, ndom);
-  if (rho) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, rho);
-  if (rho_j) {
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, rho_j);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, s, njl);
-  }
+  hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(1), 0, s, ndom, rho, rho_j, njl);
   switch (a.g.dir) {
     case 0:
       hipLaunchKernelGGL((k_line_lu<0>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, ndom, rho, jl, rho_j, njl);
