@@ -106,39 +106,41 @@ struct ash3d_tr_ctx {
   double *ofxy1 = nullptr, *ofxy2 = nullptr;
   double *dep = nullptr;
   double *fac = nullptr;  // line-solve U factors (3 * ncell)
-  // theta-scheme row factors L, R per direction (2 * ncell each), valid for lr_dt
+  // theta-scheme row factors L, R per direction (2 * ncell each), valid for
+  // lr_dt, and with them (one allocation, ln) the counts of k_line_rows, its
+  // accumulators, one INFO and one number of Jacobi sweeps per line, valid
+  // for the key (dt, theta, rmin, rmax)
   double *lr[3] = {nullptr, nullptr, nullptr};
   double lr_dt[3] = {0.0, 0.0, 0.0};
   bool lr_ok[3] = {false, false, false};
+  double *ln[3] = {nullptr, nullptr, nullptr};
+  LineCounts *ln_cnt[3] = {nullptr, nullptr, nullptr};
+  LineAcc *ln_acc[3] = {nullptr, nullptr, nullptr};
+  uint8_t *ln_jl[3] = {nullptr, nullptr, nullptr};
+  int *ln_sing[3] = {nullptr, nullptr, nullptr};
+  double ln_dt[3] = {0.0, 0.0, 0.0}, ln_th[3] = {0.0, 0.0, 0.0};
+  int ln_rmin[3] = {0, 0, 0}, ln_rmax[3] = {0, 0, 0};
+  bool ln_ok[3] = {false, false, false};
+  long long ln_count = 0;  // row factor computations launched (any direction)
   // LU factors of the theta-scheme lines per direction (one allocation:
-  // fact, D, DU, DL (4 * ncell doubles), then ncell interchange flags, one
-  // INFO per line, the count of lines that are not diagonally dominant,
-  // the largest row ratio (|DL| + |DU|) / |D| as double bits, per line the
-  // Jacobi sweeps it needs (0: more than kJacobiMaxSweepsX), the number of
-  // lines that need at most that many and their largest ratio), valid for
-  // the key (dt, theta, rmin, rmax)
+  // fact, D, DU, DL (4 * ncell doubles), then ncell interchange flags) of
+  // the same key: LU_GATED when they were left to the device to form if
+  // some line needs them (the partitioned solves' sweeps), LU_FULL when
+  // formed for the dgtsv-order solves
+  enum { LU_NONE = 0, LU_GATED = 1, LU_FULL = 2 };
   double *lu[3] = {nullptr, nullptr, nullptr};
   uint8_t *lu_piv[3] = {nullptr, nullptr, nullptr};
-  int *lu_sing[3] = {nullptr, nullptr, nullptr};
-  int *lu_ndom[3] = {nullptr, nullptr, nullptr};
-  unsigned long long *lu_rho[3] = {nullptr, nullptr, nullptr};
-  uint8_t *lu_jl[3] = {nullptr, nullptr, nullptr};
-  unsigned long long *lu_rhoj[3] = {nullptr, nullptr, nullptr};
-  int *lu_njl[3] = {nullptr, nullptr, nullptr};
-  double lu_dt[3] = {0.0, 0.0, 0.0}, lu_th[3] = {0.0, 0.0, 0.0};
-  int lu_rmin[3] = {0, 0, 0}, lu_rmax[3] = {0, 0, 0};
-  bool lu_ok[3] = {false, false, false};
-  long long lu_count = 0;  // factorisations launched (any direction)
-  // host copy of each direction's non-dominant line count (pinned, read
-  // back asynchronously after a factorisation): 0 unknown, 1 in flight
-  // (ndom_ev), 2 known.  When known, a sweep launches only the solver it
-  // needs instead of both with the choice made on the device.  The row
-  // ratios and the flagged line count come back with it (njl_h, rho_h,
-  // rhoj_h, in the same pinned block).
-  int *ndom_h = nullptr, *njl_h = nullptr;  // ndom_h: two counts per direction (k_line_lu's ndom[0], ndom[1])
-  unsigned long long *rho_h = nullptr, *rhoj_h = nullptr;
-  hipEvent_t ndom_ev[3] = {};
-  int ndom_state[3] = {0, 0, 0};
+  int lu_state[3] = {LU_NONE, LU_NONE, LU_NONE};
+  // host copy of each direction's counts (pinned; k_line_rows writes it):
+  // 0 unknown, 1 in flight (ndom_ev), 2 known.  When known, a sweep launches
+  // only the solver it needs instead of both with the choice made on the
+  // device.  The count of lines with row interchanges, which the
+  // factorisation adds later, is read back when first needed (swap_h,
+  // swap_ev, swap_state likewise).
+  LineCounts *cnt_h = nullptr;
+  int *swap_h = nullptr;
+  hipEvent_t ndom_ev[3] = {}, swap_ev[3] = {};
+  int ndom_state[3] = {0, 0, 0}, swap_state[3] = {0, 0, 0};
   bool capturing = false;
   // the velocity ghosts hold Set_BC(1)'s values for the current interior
   // velocities (cleared by every entry point that writes velocities)
@@ -163,8 +165,9 @@ struct ash3d_tr_ctx {
   // brings the caches back to them before a replay)
   DiffArgs lu_args[3] = {};
   bool lu_args_set[3] = {false, false, false};
+  bool lu_args_full[3] = {false, false, false};  // the dgtsv-order solves may read the factors
   DiffArgs graph_lu[2][3] = {};
-  bool graph_lu_on[2][3] = {};
+  bool graph_lu_on[2][3] = {}, graph_lu_full[2][3] = {};
   bool graph_tgeom[2] = {false, false};  // the graph reads the transposed geometry
   long long fac_groups = 0;
   double *flux = nullptr;  // source column staging (nz+1)*ns
@@ -494,58 +497,95 @@ int ensure_tgeom(ash3d_tr_ctx *x) {
   return 0;
 }
 
-// Row factors L, R of the theta-scheme lines of one direction, recomputed
-// when dt changes (the geometry and K uploads invalidate them)
+// Row factors L, R of the theta-scheme lines of one direction and the
+// counts of its active range
+int run_line_rows(ash3d_tr_ctx *x, int dir, const DiffArgs &a) {
+  int rc = 0;
+  const long long lines = (long long)a.g.Na * a.g.Nb;
+  constexpr long long kHead = (sizeof(LineCounts) + sizeof(LineAcc)) / sizeof(double);
+  if (!x->ln[dir]) {
+    if ((rc = dev_alloc(&x->ln[dir], kHead + (lines + 1) / 2 + (lines + 7) / 8))) return rc;
+    x->ln_cnt[dir] = (LineCounts *)x->ln[dir];
+    x->ln_acc[dir] = (LineAcc *)(x->ln_cnt[dir] + 1);
+    x->ln_sing[dir] = (int *)(x->ln_acc[dir] + 1);
+    x->ln_jl[dir] = (uint8_t *)(x->ln[dir] + kHead + (lines + 1) / 2);
+    HIPCHK(launch_fill(x->stream, x->ln[dir], kHead, 0.0));
+  }
+  if (!x->cnt_h && hipHostMalloc((void **)&x->cnt_h, 3 * (sizeof(LineCounts) + sizeof(int)), hipHostMallocDefault) !=
+                       hipSuccess) {
+    x->cnt_h = nullptr;  // (the counts stay unknown to the host)
+    (void)hipGetLastError();
+  }
+  if (x->cnt_h) x->swap_h = (int *)(x->cnt_h + 3);
+  const LineStats st{x->ln_acc[dir], x->ln_cnt[dir], x->cnt_h ? x->cnt_h + dir : nullptr, x->ln_jl[dir],
+                     x->ln_sing[dir]};
+  HIPCHK(launch_line_rows(x->stream, a, x->lr[dir], st));
+  x->lr_ok[dir] = x->ln_ok[dir] = true;
+  x->lr_dt[dir] = x->ln_dt[dir] = a.dt;
+  x->ln_th[dir] = a.theta;
+  x->ln_rmin[dir] = a.g.rmin;
+  x->ln_rmax[dir] = a.g.rmax;
+  x->lu_state[dir] = ash3d_tr_ctx::LU_NONE;
+  x->swap_state[dir] = 0;
+  return 0;
+}
+
+// Row factors of the lines of one direction, recomputed when dt changes
+// (the geometry and K uploads invalidate them)
 int ensure_lr(ash3d_tr_ctx *x, int dir, DiffArgs &a) {
   int rc = 0;
   if (!x->lr[dir] && (rc = dev_alloc(&x->lr[dir], 2 * x->d.ncell))) return rc;
   if (!x->lr_ok[dir] || x->lr_dt[dir] != a.dt) {
-    HIPCHK(launch_line_lr(x->stream, a, x->lr[dir]));
-    x->lr_ok[dir] = true;
-    x->lr_dt[dir] = a.dt;
-    x->lu_ok[dir] = false;
+    if ((rc = run_line_rows(x, dir, a))) return rc;
+    ++x->ln_count;
+    x->ndom_state[dir] = 0;
   }
   a.lr = x->lr[dir];
   return 0;
 }
 
-// LU factors of the theta-scheme lines of one direction (after ensure_lr),
-// refactored when dt, theta or the active range along the lines changes
-int ensure_lu(ash3d_tr_ctx *x, int dir, DiffArgs &a) {
+// A sweep of n active cells whose lines the dgtsv-order solves may take
+// whatever the lines are
+bool dgtsv_sweep(const ash3d_tr_ctx *x, int dir, int n) {
+  const int nmax = dir == 0 ? x->part_max_line : x->part_max_line_strided;
+  return x->line_solver != ASH3D_LINE_SOLVER_PARTITIONED || n < 3 || n > nmax;
+}
+
+// Counts and LU factors of the theta-scheme lines of one direction (after
+// ensure_lr), renewed when dt, theta or the active range along the lines
+// changes.  full: the dgtsv-order solves may read the factors of any line;
+// otherwise the partitioned solves take the sweep unless a line is not
+// dominant, and the device forms the factors only if some line needs them.
+int ensure_lu(ash3d_tr_ctx *x, int dir, DiffArgs &a, bool full) {
   int rc = 0;
-  const long long nc = x->d.ncell, lines = (long long)a.g.Na * a.g.Nb;
+  const long long nc = x->d.ncell;
   if (!x->lu[dir]) {
-    const long long tail = 4 * nc + (nc + 7) / 8 + (lines + 1) / 2;
-    if ((rc = dev_alloc(&x->lu[dir], tail + 4 + (lines + 7) / 8))) return rc;
+    if ((rc = dev_alloc(&x->lu[dir], 4 * nc + (nc + 7) / 8))) return rc;
     x->lu_piv[dir] = (uint8_t *)(x->lu[dir] + 4 * nc);
-    x->lu_sing[dir] = (int *)(x->lu[dir] + 4 * nc + (nc + 7) / 8);
-    x->lu_ndom[dir] = (int *)(x->lu[dir] + tail);
-    x->lu_rho[dir] = (unsigned long long *)(x->lu[dir] + tail + 1);
-    x->lu_rhoj[dir] = (unsigned long long *)(x->lu[dir] + tail + 2);
-    x->lu_njl[dir] = (int *)(x->lu[dir] + tail + 3);
-    x->lu_jl[dir] = (uint8_t *)(x->lu[dir] + tail + 4);
   }
   if (!x->junk && (rc = dev_alloc(&x->junk, kJunk))) return rc;
-  if (!x->lu_ok[dir] || x->lu_dt[dir] != a.dt || x->lu_th[dir] != a.theta || x->lu_rmin[dir] != a.g.rmin ||
-      x->lu_rmax[dir] != a.g.rmax) {
-    HIPCHK(launch_line_lu(x->stream, a, x->lu[dir], x->lu_piv[dir], x->lu_sing[dir], x->lu_ndom[dir],
-                          x->lu_rho[dir], x->lu_jl[dir], x->lu_rhoj[dir], x->lu_njl[dir]));
-    ++x->lu_count;
+  if (!x->ln_ok[dir] || x->ln_dt[dir] != a.dt || x->ln_th[dir] != a.theta || x->ln_rmin[dir] != a.g.rmin ||
+      x->ln_rmax[dir] != a.g.rmax) {
+    if ((rc = run_line_rows(x, dir, a))) return rc;
+    ++x->ln_count;
     x->ndom_state[dir] = 0;
-    x->lu_ok[dir] = true;
-    x->lu_dt[dir] = a.dt;
-    x->lu_th[dir] = a.theta;
-    x->lu_rmin[dir] = a.g.rmin;
-    x->lu_rmax[dir] = a.g.rmax;
+  }
+  const int want = full ? ash3d_tr_ctx::LU_FULL : ash3d_tr_ctx::LU_GATED;
+  if (x->lu_state[dir] < want) {
+    // (gated factors to be completed: the counts start over at the same values)
+    if (x->lu_state[dir] != ash3d_tr_ctx::LU_NONE && (rc = run_line_rows(x, dir, a))) return rc;
+    HIPCHK(launch_line_lu(x->stream, a, x->lu[dir], x->lu_piv[dir], x->ln_sing[dir], x->ln_cnt[dir], !full));
+    x->lu_state[dir] = want;
   }
   a.lu = x->lu[dir];
   a.piv = x->lu_piv[dir];
-  a.sing = x->lu_sing[dir];
-  a.ndom = x->lu_ndom[dir];
+  a.sing = x->ln_sing[dir];
+  a.ndom = &x->ln_cnt[dir]->ndom;
   a.sel = 0;
   a.junk = x->junk;
   x->lu_args[dir] = a;
   x->lu_args_set[dir] = true;
+  x->lu_args_full[dir] = full;
   return 0;
 }
 
@@ -571,31 +611,13 @@ int ensure_fac(ash3d_tr_ctx *x, int nb) {
 // factorisation, and always inside a graph capture, whose sweeps keep the
 // device-side choice so that a replay after a refactorisation is right).
 int host_ndom(ash3d_tr_ctx *x, int dir) {
-  if (x->capturing || !x->lu_ok[dir]) return -1;
+  if (x->capturing || !x->ln_ok[dir] || !x->cnt_h) return -1;
   if (x->ndom_state[dir] == 0) {
-    if (!x->ndom_h) {
-      if (hipHostMalloc((void **)&x->ndom_h, 128, hipHostMallocDefault) != hipSuccess) {
-        x->ndom_h = nullptr;
-        return -1;
-      }
-      x->njl_h = x->ndom_h + 6;
-      x->rho_h = (unsigned long long *)(x->ndom_h + 10);
-      x->rhoj_h = x->rho_h + 3;
-    }
     if (!x->ndom_ev[dir] && hipEventCreateWithFlags(&x->ndom_ev[dir], hipEventDisableTiming) != hipSuccess) {
       x->ndom_ev[dir] = nullptr;
       return -1;
     }
-    if (hipMemcpyAsync(x->ndom_h + 2 * dir, x->lu_ndom[dir], 2 * sizeof(int), hipMemcpyDeviceToHost, x->stream) !=
-            hipSuccess ||
-        hipMemcpyAsync(x->rho_h + dir, x->lu_rho[dir], sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                       x->stream) != hipSuccess ||
-        hipMemcpyAsync(x->rhoj_h + dir, x->lu_rhoj[dir], sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                       x->stream) != hipSuccess ||
-        hipMemcpyAsync(x->njl_h + dir, x->lu_njl[dir], sizeof(int), hipMemcpyDeviceToHost, x->stream) !=
-            hipSuccess ||
-        hipEventRecord(x->ndom_ev[dir], x->stream) != hipSuccess)
-      return -1;
+    if (hipEventRecord(x->ndom_ev[dir], x->stream) != hipSuccess) return -1;
     x->ndom_state[dir] = 1;
     return -1;
   }
@@ -603,11 +625,31 @@ int host_ndom(ash3d_tr_ctx *x, int dir) {
     if (hipEventQuery(x->ndom_ev[dir]) != hipSuccess) return -1;
     x->ndom_state[dir] = 2;
   }
-  return x->ndom_h[2 * dir];
+  return x->cnt_h[dir].ndom;
 }
 
-// the same for the count of lines whose elimination interchanges rows
-int host_nswap(ash3d_tr_ctx *x, int dir) { return host_ndom(x, dir) < 0 ? -1 : x->ndom_h[2 * dir + 1]; }
+// the same for the count of lines whose elimination interchanges rows, of
+// factors that were formed
+int host_nswap(ash3d_tr_ctx *x, int dir) {
+  if (x->capturing || !x->ln_ok[dir] || !x->cnt_h) return -1;
+  if (x->swap_state[dir] == 0) {
+    if (!x->swap_ev[dir] && hipEventCreateWithFlags(&x->swap_ev[dir], hipEventDisableTiming) != hipSuccess) {
+      x->swap_ev[dir] = nullptr;
+      return -1;
+    }
+    if (hipMemcpyAsync(x->swap_h + dir, &x->ln_cnt[dir]->nswap, sizeof(int), hipMemcpyDeviceToHost, x->stream) !=
+            hipSuccess ||
+        hipEventRecord(x->swap_ev[dir], x->stream) != hipSuccess)
+      return -1;
+    x->swap_state[dir] = 1;
+    return -1;
+  }
+  if (x->swap_state[dir] == 1) {
+    if (hipEventQuery(x->swap_ev[dir]) != hipSuccess) return -1;
+    x->swap_state[dir] = 2;
+  }
+  return x->swap_h[dir];
+}
 
 // Jacobi sweeps for a theta-scheme sweep of y or z lines that would
 // otherwise be solved in dgtsv order (partitioned mode, eager steps): the
@@ -628,7 +670,7 @@ int jacobi_iters(ash3d_tr_ctx *x, int dir) {
   if (dir == 0 || x->line_solver != ASH3D_LINE_SOLVER_PARTITIONED || x->jacobi_sweeps <= 0) return -1;
   if (host_ndom(x, dir) != 0) return -1;
   double rho;
-  std::memcpy(&rho, x->rho_h + dir, sizeof rho);
+  std::memcpy(&rho, &x->cnt_h[dir].rho, sizeof rho);
   return jacobi_k(rho, x->jacobi_sweeps);
 }
 
@@ -643,9 +685,9 @@ int jacobi_iters(ash3d_tr_ctx *x, int dir) {
 int jacobi_x_sweeps(ash3d_tr_ctx *x, int n) {
   if (x->line_solver != ASH3D_LINE_SOLVER_PARTITIONED || x->jacobi_sweeps <= 0 || x->jacobi_x == 0) return 0;
   if (n < 3 || n > x->part_max_line || (x->jacobi_x == 1 && n < 256)) return 0;
-  if (host_ndom(x, 0) != 0 || x->njl_h[0] == 0) return 0;
+  if (host_ndom(x, 0) != 0 || x->cnt_h[0].njl == 0) return 0;
   double rho;
-  std::memcpy(&rho, x->rhoj_h, sizeof rho);
+  std::memcpy(&rho, &x->cnt_h[0].rho_j, sizeof rho);
   const int sw = jacobi_sweeps_needed(rho, kJacobiMaxSweepsX);
   return sw == 0 ? 0 : std::min(sw, x->jacobi_sweeps);
 }
@@ -684,8 +726,7 @@ int try_cn_partitioned(ash3d_tr_ctx *x, int dir, DiffArgs &a, int *rc, bool adjo
   // (x lines are contiguous in memory; y and z lines strided; the adjoint's
   // partitioned solves take the lines the forward's took, so that the
   // sweeps the forward ran as Jacobi sweeps get their transpose)
-  const int nmax = dir == 0 ? x->part_max_line : x->part_max_line_strided;
-  if (x->line_solver != ASH3D_LINE_SOLVER_PARTITIONED || n < 3 || n > nmax) return 0;
+  if (dgtsv_sweep(x, dir, n)) return 0;
   const int hn = host_ndom(x, dir);
   if (hn > 0) return 0;
   const PartLayout lay = part_layout(x, dir, a);
@@ -772,7 +813,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
     const Dims &d = x->d;
     if ((rc = ensure_tgeom(x))) return rc;
     transpose_x_args(x, bounds, a);
-    if ((rc = ensure_lr(x, 0, a)) || (rc = ensure_lu(x, 0, a))) return rc;
+    if ((rc = ensure_lr(x, 0, a)) || (rc = ensure_lu(x, 0, a, dgtsv_sweep(x, 0, a.g.rmax - a.g.rmin + 1)))) return rc;
     {
       ProfScope ps(x, ASH3D_PROF_DIFFUSE_X);  // one record for the kernels
       const int sw = jacobi_x_sweeps(x, a.g.rmax - a.g.rmin + 1);
@@ -781,7 +822,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
         // the lines that need at most jacobi_sweeps sweeps, then the
         // partitioned solves of the others (which certainly run: every
         // line dominant, n in range)
-        a.jline = x->lu_jl[0];
+        a.jline = x->ln_jl[0];
         a.jcap = x->jacobi_sweeps;
         HIPCHK(launch_diff_cn_jacobi_x(x->stream, a, d, x->ts0(), x->kap, x->sx, x->kx));
       }
@@ -794,7 +835,8 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
     return 0;
   }
   if (use_cn) {
-    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a))) return rc;
+    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, dgtsv_sweep(x, dir, a.g.rmax - a.g.rmin + 1))))
+      return rc;
     ProfScope ps(x, ASH3D_PROF_DIFFUSE_X + dir);  // one record for both kernels
     const int tp = try_cn_partitioned(x, dir, a, &rc);
     if (rc) return rc;
@@ -868,7 +910,8 @@ int adj_diffuse_sweep(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double im
   // once on the device when those ran
   const int *skip = nullptr;
   if (use_cn && x->line_solver == ASH3D_LINE_SOLVER_PARTITIONED) {
-    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a))) return rc;
+    // (the dgtsv-order transposes form their own factors)
+    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, false))) return rc;
     a.c0 = x->lam;
     ProfScope ps(x, ASH3D_PROF_ADJ_DIFFUSE);
     const int n = a.g.rmax - a.g.rmin + 1;
@@ -879,7 +922,7 @@ int adj_diffuse_sweep(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double im
       const int sw = jacobi_x_sweeps(x, n);
       x->jacobi_last[0] = sw;
       if (sw > 0) {
-        a.jline = x->lu_jl[0];
+        a.jline = x->ln_jl[0];
         a.jcap = x->jacobi_sweeps;
         HIPCHK(launch_diff_cn_jacobi_x(x->stream, a, x->d, x->lam, x->kap, x->sx, x->kx, true));
       }
@@ -1029,7 +1072,7 @@ int ash3d_tr_destroy(ash3d_tr_ctx *x) {
                     x->ddx, x->ddy, x->ofxz1, x->ofxz2, x->ofyz1, x->ofyz2, x->ofxy1, x->ofxy2, x->dep,
                     x->fac, x->flux, x->tot, x->tq, x->tkap, x->tsx, x->tkx, x->lam, x->snap_b,
                     x->snap_z, x->adj_sb, x->sink, x->src_grad, x->col, x->lr[0], x->lr[1], x->lr[2],
-                    x->lu[0], x->lu[1], x->lu[2], x->junk, x->prod, x->dtvc};
+                    x->lu[0], x->lu[1], x->lu[2], x->ln[0], x->ln[1], x->ln[2], x->junk, x->prod, x->dtvc};
   for (double *p : ptrs)
     if (p) hipFree(p);
   for (double *p : x->ckpt)
@@ -1046,15 +1089,17 @@ int ash3d_tr_destroy(ash3d_tr_ctx *x) {
     if (x->flux_ev[k]) hipEventDestroy(x->flux_ev[k]);
   }
   if (x->flag) hipFree(x->flag);
-  if (x->ndom_h) hipHostFree(x->ndom_h);
+  if (x->cnt_h) hipHostFree(x->cnt_h);
   if (x->umb_src) hipFree(x->umb_src);
   if (x->umb_wind) hipFree(x->umb_wind);
   for (int k = 0; k < 2; ++k) {
     if (x->umb_pin[k]) hipHostFree(x->umb_pin[k]);
     if (x->umb_ev[k]) hipEventDestroy(x->umb_ev[k]);
   }
-  for (int k = 0; k < 3; ++k)
+  for (int k = 0; k < 3; ++k) {
     if (x->ndom_ev[k]) hipEventDestroy(x->ndom_ev[k]);
+    if (x->swap_ev[k]) hipEventDestroy(x->swap_ev[k]);
+  }
   for (auto &e : x->ev_pool) {
     hipEventDestroy(e.first);
     hipEventDestroy(e.second);
@@ -1975,6 +2020,7 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
   for (int k = 0; k < 3; ++k) {
     x->graph_lu_on[slot][k] = x->lu_args_set[k];
     x->graph_lu[slot][k] = x->lu_args[k];
+    x->graph_lu_full[slot][k] = x->lu_args_full[k];
   }
   x->graph_tgeom[slot] = use_diffusion && use_cn;
   return 0;
@@ -1994,7 +2040,7 @@ int ash3d_tr_graph_launch(ash3d_tr_ctx *x, int32_t itime) {
   for (int k = 0; k < 3; ++k) {
     if (!x->graph_lu_on[slot][k]) continue;
     DiffArgs a = x->graph_lu[slot][k];
-    if ((rc = ensure_lr(x, k, a)) || (rc = ensure_lu(x, k, a))) return rc;
+    if ((rc = ensure_lr(x, k, a)) || (rc = ensure_lu(x, k, a, x->graph_lu_full[slot][k]))) return rc;
   }
   HIPCHK(hipGraphLaunch(x->graph[slot], x->stream));
   x->ts1_state = TS1_MIRROR;
@@ -2253,7 +2299,7 @@ int ens_prepare(ash3d_tr_ctx *x, double dt, double imp_fac, const int32_t *is_al
                 bool *refactored = nullptr) {
   int rc = check_ctx_keep(x);
   if (rc) return rc;
-  const long long lu_before = x->lu_count;
+  const long long lu_before = x->ln_count;
   // after a step (ts1 mirrored) the ensemble step's glue only zeroes ghost
   // cells the step rewrites; after a glue (ts1 zero) the member steps from
   // ts0 as it is
@@ -2275,9 +2321,9 @@ int ens_prepare(ash3d_tr_ctx *x, double dt, double imp_fac, const int32_t *is_al
     if (n < 3 || n > std::min(nmax, 2048))
       return fail(ASH3D_TR_EINVAL, "ensemble member: %d active cells along dir %d (partitioned solves take 3..%d)",
                   n, dir, std::min(nmax, 2048));
-    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a))) return rc;
+    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, false))) return rc;
   }
-  if (refactored) *refactored = x->lu_count != lu_before;
+  if (refactored) *refactored = x->ln_count != lu_before;
   return 0;
 }
 
@@ -2288,7 +2334,7 @@ int ens_check_dominant(ash3d_tr_ctx *x, size_t k) {
   HIPCHK(hipStreamSynchronize(x->stream));
   for (int dir = 0; dir < 3; ++dir) {
     int h = 0;
-    HIPCHK(hipMemcpy(&h, x->lu_ndom[dir], sizeof(int), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(&h, &x->ln_cnt[dir]->ndom, sizeof(int), hipMemcpyDeviceToHost));
     if (h != 0)
       return fail(ASH3D_TR_EINVAL, "ensemble member %zu: %d lines along dir %d are not diagonally dominant", k, h, dir);
   }
@@ -2337,7 +2383,7 @@ int ens_member_specs(ash3d_tr_ctx *x, int itime, double dt, double imp_fac, cons
     else spec_neumann_dir(x->d, dir, x->periodic, x->ts0(), &slots[q++]);
     DiffArgs a = diff_args(x, dir, dt, imp_fac, is_aloft, b);
     if (dir == 0) transpose_x_args(x, b, a);
-    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a))) return rc;
+    if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, false))) return rc;
     a.sel = 1;
     hipError_t e = spec_diff_cn_part(a, part_layout(x, dir, a), x->part_bins, x->part_shape[dir], &slots[q++]);
     if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "ensemble diffusion dir %d: %s", dir, hipGetErrorString(e));

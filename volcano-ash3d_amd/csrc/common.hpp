@@ -175,15 +175,15 @@ struct DiffArgs {
   const uint8_t *piv;
   const int *sing;
   // number of lines of the sweep whose matrix is not diagonally dominant
-  // (from k_line_lu) and, in ndom[1], of lines whose elimination interchanges
-  // rows; sel = 1: the partitioned solves run only when ndom[0] is zero,
+  // and, in ndom[1], of lines whose elimination interchanges rows (the first
+  // two of LineCounts); sel = 1: the partitioned solves run only when ndom[0] is zero,
   // sel = 2: only when it is not (their dgtsv-order alternative), sel = 3
   // and 4: the dgtsv-order kernels with, and without, row interchanges only
   // when ndom[1] is not zero, and zero; sel = 0: always
   const int *ndom;
   int sel;
   double *junk;        // kJunk doubles that masked-off lanes store to
-  // per line of the sweep (k_line_lu's line index): the Jacobi sweeps the
+  // per line of the sweep (k_line_rows' line index): the Jacobi sweeps the
   // line needs (0: more than kJacobiMaxSweepsX); lines with 1 <= jline <= jcap are
   // solved by the Jacobi sweeps and skipped by the partitioned solves.
   // null: none
@@ -289,8 +289,34 @@ hipError_t launch_diff_cn(hipStream_t s, const DiffArgs &a, int nb);
 // kernel returns at once when a.ndom[1] is not zero).  x lines: a describes the x<->y
 // transposed grid, orig and c_orig the state; otherwise null
 hipError_t launch_cn_exact(hipStream_t s, const DiffArgs &a, const Dims *orig, double *c_orig);
+// What the choice of a sweep's solver needs to know of its lines: how many
+// are not diagonally dominant M-matrix rows, have a row interchange in
+// dgtsv's elimination (known once k_line_lu ran), may need that elimination
+// although they count as dominant or not (nlu), need at most
+// kJacobiMaxSweepsX Jacobi sweeps (njl); the largest row ratio
+// (|DL| + |DU|) / |D| as double bits, 1.0 when a line is not dominant, and
+// the largest among the njl lines
+struct LineCounts {
+  int ndom, nswap, nlu, njl;
+  unsigned long long rho, rho_j;
+};
+// accumulators of one launch (zero between launches)
+struct LineAcc {
+  int ndom, nlu, njl, done;
+  unsigned long long rho, rho_j;
+};
+// jl[line]: the Jacobi sweeps the line needs (jacobi_sweeps_needed of its
+// ratio; 0: more than kJacobiMaxSweepsX); sing[line] is cleared; *res and,
+// if not null, *host (pinned) receive the counts
+struct LineStats {
+  LineAcc *acc;
+  LineCounts *res, *host;
+  uint8_t *jl;
+  int *sing;
+};
 // the row factors L, R of every cell of the sweep's lines (bin-independent)
-hipError_t launch_line_lr(hipStream_t s, const DiffArgs &a, double *lr);
+// and the LineStats of the active range
+hipError_t launch_line_rows(hipStream_t s, const DiffArgs &a, double *lr, const LineStats &st);
 // partitioned line solves (linesolve.hip): offsets of cell r of line (a, b)
 // are st0 + sta*a + stb*b + str*r in the state and lr0 + lra*a + lrb*b +
 // lrr*r in the row factor cache (R at + lr_ncell); hipErrorInvalidValue
@@ -306,15 +332,10 @@ hipError_t launch_diff_cn_part(hipStream_t s, const DiffArgs &a, const PartLayou
                                bool adjoint = false);
 // the launch of the forward partitioned solves (launch_diff_cn_part)
 hipError_t spec_diff_cn_part(const DiffArgs &a, const PartLayout &lay, int bins_wg, int shape, LaunchSpec *sp);
-// the LU factors of every line of the sweep (reads a.lr)
-// (*rho: the largest row ratio (|DL| + |DU|) / |D| over the sweep's lines as
-// double bits, 1.0 when a line is not diagonally dominant; may be null.
-// jl[line]: the Jacobi sweeps the line needs (jacobi_sweeps_needed of its
-// ratio; 0: more than kJacobiMaxSweepsX), *rho_j the largest ratio of the
-// lines that need at most that many and *njl their number; all three null
-// or all given)
-hipError_t launch_line_lu(hipStream_t s, const DiffArgs &a, double *lu, uint8_t *piv, int *sing, int *ndom,
-                          unsigned long long *rho, uint8_t *jl, unsigned long long *rho_j, int *njl);
+// the LU factors of every line of the sweep (reads a.lr), after
+// launch_line_rows; gated: the kernel returns at once when cnt->nlu is zero
+hipError_t launch_line_lu(hipStream_t s, const DiffArgs &a, double *lu, uint8_t *piv, int *sing, LineCounts *cnt,
+                          bool gated);
 // theta-scheme solves of y or z lines by K + 1 Jacobi sweeps (0 <= k <=
 // kJacobiMaxIters), in one pass, for sweeps whose rows are all diagonally
 // dominant (nb: bins per thread, 1, 2 or 4)

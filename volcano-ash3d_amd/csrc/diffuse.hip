@@ -22,38 +22,137 @@ namespace {
 
 constexpr int kBlock = 256;
 
-// Row factors of the theta-scheme lines, one thread per cell (lanes along
-// the contiguous transverse index).  For the row of cell c (:807-816):
+// Rows of the theta-scheme lines.  For the row of cell c (:807-816):
 //   kds_I = (0.5*(K_{I-1}+K_I)) * (sig_I / (0.5*(kap_{I-1}+kap_I)))
 //   L = dt*kds_c*sig_c/kap_c,  R = dt*kds_{c+1}*sig_{c+1}/kap_c
 // They depend on dt, the geometry and K only, so the context keeps them
 // between steps; the line solves then read two numbers per row instead of
 // evaluating three divisions in every bin group.
-template <int DIR>
-__global__ __launch_bounds__(kBlock) void k_line_lr(DiffArgs A, double *lr) {
+//
+// With them come, from the rows of the active range [rmin, rmax], what the
+// choice of the solver needs to know of the matrix (LineStats): which lines
+// are not diagonally dominant M-matrix rows (some L or R negative or not
+// finite, or theta < 0: the partitioned solves, which eliminate without
+// pivoting, take none), the largest row ratio (|DL| + |DU|) / |D|, and per
+// line the Jacobi sweeps it needs.
+//
+// A workgroup is 64 lines (lanes along the contiguous transverse index) by
+// W runs of rows, one per wave, each keeping the face it shares with the
+// next row; per-line results meet in LDS, the sweep's in one set of atomics
+// per workgroup, and the last workgroup to finish publishes them and clears
+// the accumulators.  Bound by reading kappa, K and sigma and writing L and
+// R (40 B per cell): 63 us at 360x240x50, where a pass over the cells for L
+// and R (58 us) and the serial factorisation that found the ratios (61 us
+// along z, 198 us along x and y) took 119 to 256 us for each new time step.
+constexpr double kSafeRatio = 1.0 - 0x1p-20;
+
+template <int DIR, int W>
+__global__ __launch_bounds__(64 * W) void k_line_rows(DiffArgs A, double *lr, LineStats S) {
   const Dims d = A.d;
   const LineGeom g = A.g;
-  const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= (long long)g.Na * g.N * g.Nb) return;
-  const int a = (int)(t % g.Na) + 1;
-  const long long rest = t / g.Na;
-  const int r = (int)(rest % g.N) + 1;
-  const int b = (int)(rest / g.N) + 1;
-  const long long sL = line_stride(d, DIR), base = line_base(d, DIR, a, b);
-  const long long kS = kline_stride(d, DIR), kB = kline_base(d, DIR, a, b);
-  auto kapat = [&](int q) { return A.kap[base + sL * (long long)(q + 1)]; };
-  auto Kat = [&](int q) { return A.kk[kB + kS * (long long)q]; };
-  auto sigat = [&](int q) { return A.sig[base + sL * (long long)(q + 1)]; };
-  auto kds_at = [&](int I) {
-    const double vavg = 0.5 * (kapat(I - 1) + kapat(I));
-    const double kavg = 0.5 * (Kat(I - 1) + Kat(I));
-    const double ds = sigat(I) / vavg;
-    return kavg * ds;
-  };
-  const double dt = A.dt, kap_c = kapat(r);
-  const long long o = base + sL * (long long)(r + 1);
-  lr[o] = dt * kds_at(r) * sigat(r) / kap_c;
-  lr[o + d.ncell] = dt * kds_at(r + 1) * sigat(r + 1) / kap_c;
+  const long long lines = (long long)g.Na * g.Nb;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long gid = (long long)blockIdx.x * 64 + lane;
+  const bool on = gid < lines;
+  const int N = g.N, run = (N + W - 1) / W;
+  const int r0 = 1 + w * run, r1 = min(N, r0 + run - 1);
+  const double th = A.theta;
+  bool dom = true;
+  double rho = 0.0;  // largest (|DL| + |DU|) / |D| of the rows
+  if (on && r0 <= r1) {
+    const int a = (int)(gid % g.Na) + 1;
+    const int b = (int)(gid / g.Na) + 1;
+    const long long sL = line_stride(d, DIR), kS = kline_stride(d, DIR);
+    const double *kap = A.kap + line_base(d, DIR, a, b) + sL;  // of cell q at sL * q
+    const double *sig = A.sig + line_base(d, DIR, a, b) + sL;
+    const double *kk = A.kk + kline_base(d, DIR, a, b);
+    double *lo = lr + line_base(d, DIR, a, b) + sL;
+    double kap_l = kap[sL * (r0 - 1)], k_l = kk[kS * (r0 - 1)];
+    double kap_c = kap[sL * r0], k_c = kk[kS * r0], sig_c = sig[sL * r0];
+    double kds_c = 0.5 * (k_l + k_c) * (sig_c / (0.5 * (kap_l + kap_c)));
+#pragma unroll 4
+    for (int r = r0; r <= r1; ++r) {
+      const double kap_r = kap[sL * (r + 1)], k_r = kk[kS * (r + 1)], sig_r = sig[sL * (r + 1)];
+      const double kds_r = 0.5 * (k_c + k_r) * (sig_r / (0.5 * (kap_c + kap_r)));
+      const double L = A.dt * kds_c * sig_c / kap_c;
+      const double R = A.dt * kds_r * sig_r / kap_c;
+      lo[sL * r] = L;
+      lo[sL * r + d.ncell] = R;
+      if (r >= g.rmin && r <= g.rmax) {
+        const double C = L + R;
+        double D = 1.0 + th * C, DL = 0.0, DU = 0.0;
+        if (r > g.rmin) DL = -(th * L);
+        if (r < g.rmax) DU = -(th * R);
+        if (r == g.rmin) D = D - th * L;
+        else if (r == g.rmax) D = D - th * R;
+        // L, R >= 0 and finite, theta >= 0: every row has D >= 1 + |DL| + |DU|
+        // in exact arithmetic (false for NaN too)
+        dom = dom && L >= 0.0 && R >= 0.0 && L <= DBL_MAX && R <= DBL_MAX && th >= 0.0;
+        rho = fmax(rho, (fabs(DL) + fabs(DU)) / fabs(D));
+      }
+      kap_c = kap_r;
+      k_c = k_r;
+      sig_c = sig_r;
+      kds_c = kds_r;
+    }
+  }
+  __shared__ double s_rho[W][64];
+  __shared__ unsigned long long s_ndom[W];
+  s_rho[w][lane] = rho;
+  // lines with a row that is not dominant, as one bit mask per run of rows
+  const unsigned long long nd = __ballot(!dom);
+  if (lane == 0) s_ndom[w] = nd;
+  __syncthreads();
+  if (w != 0) return;
+  unsigned long long bad = 0;
+#pragma unroll
+  for (int q = 0; q < W; ++q) {
+    rho = fmax(rho, s_rho[q][lane]);
+    bad |= s_ndom[q];
+  }
+  dom = !((bad >> lane) & 1);
+  const double r = !on ? 0.0 : ((dom && rho < 1.0) ? rho : 1.0);
+  const int sw = (on && dom) ? jacobi_sweeps_needed(r, kJacobiMaxSweepsX) : 0;
+  if (on) {
+    S.jl[gid] = (uint8_t)sw;
+    S.sing[gid] = 0;
+  }
+  // rows whose elimination may meet a zero pivot or that are not dominant
+  // (a ratio of at most kSafeRatio leaves every pivot, of either row order,
+  // larger than the rest of its row by that margin)
+  const int n_dom = __popcll(__ballot(on && !dom)), n_lu = __popcll(__ballot(on && !(r <= kSafeRatio)));
+  const int n_j = __popcll(__ballot(sw > 0));
+  double rmax = r, jmax = sw > 0 ? r : 0.0;
+  for (int o = 32; o; o >>= 1) {
+    rmax = fmax(rmax, __shfl_xor(rmax, o));
+    jmax = fmax(jmax, __shfl_xor(jmax, o));
+  }
+  if (lane != 0) return;
+  // (non-negative doubles order as their bit patterns)
+  if (n_dom) atomicAdd(&S.acc->ndom, n_dom);
+  if (n_lu) atomicAdd(&S.acc->nlu, n_lu);
+  if (n_j) atomicAdd(&S.acc->njl, n_j);
+  atomicMax(&S.acc->rho, (unsigned long long)__double_as_longlong(rmax));
+  if (n_j) atomicMax(&S.acc->rho_j, (unsigned long long)__double_as_longlong(jmax));
+  // the accumulators are touched by device-scope atomics only, so their
+  // completion is all that the count of finished workgroups has to follow (a
+  // fence would write back the L2 that holds the row factors)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (atomicAdd(&S.acc->done, 1) != (int)gridDim.x - 1) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  LineCounts c;
+  c.ndom = atomicExch(&S.acc->ndom, 0);
+  c.nswap = 0;
+  c.nlu = atomicExch(&S.acc->nlu, 0);
+  c.njl = atomicExch(&S.acc->njl, 0);
+  c.rho = atomicExch(&S.acc->rho, 0ull);
+  c.rho_j = atomicExch(&S.acc->rho_j, 0ull);
+  atomicExch(&S.acc->done, 0);
+  *S.res = c;
+  if (S.host) {
+    *S.host = c;
+    __threadfence_system();
+  }
 }
 
 // LU factorisation of the theta-scheme lines: dgtsv's elimination
@@ -65,15 +164,15 @@ __global__ __launch_bounds__(kBlock) void k_line_lr(DiffArgs A, double *lr) {
 // interchange flag piv_i of elimination step i (rows i and i+1), and the U
 // entries D_i, DU_i, DL_i (DL_i: second super-diagonal); D_n on the last
 // row.  sing[line] is dgtsv's INFO for the line (first zero pivot row).
-// *ndom counts the lines that are not diagonally dominant M-matrix rows
-// (some L or R negative or not finite, or theta < 0): the partitioned
-// solves, which eliminate without pivoting, are used only when it is zero.
-// ndom[1] counts the lines with an interchange (a row dominant in itself is
-// interchanged when the next row's sub-diagonal entry is larger still).
+// cnt->nswap counts the lines with an interchange (a row dominant in itself
+// is interchanged when the next row's sub-diagonal entry is larger still).
+// gated: run only if some line may need the factors although the
+// partitioned solves are the sweep's (cnt->nlu, from k_line_rows): the usual
+// sweep, whose lines are all dominant, pays 4 us for the look.
 template <int DIR>
-__global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint8_t *piv, int *sing, int *ndom,
-                                                   unsigned long long *rho, uint8_t *jl, unsigned long long *rho_j,
-                                                   int *njl) {
+__global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint8_t *piv, int *sing, LineCounts *cnt,
+                                                   bool gated) {
+  if (gated && cnt->nlu == 0) return;
   const Dims d = A.d;
   const LineGeom g = A.g;
   const long long gid = (long long)blockIdx.x * kBlock + threadIdx.x;
@@ -86,8 +185,7 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
   const double *Lf = A.lr, *Rf = A.lr + d.ncell;
   double *fF = lu, *fD = lu + d.ncell, *fDU = fD + d.ncell, *fDL = fDU + d.ncell;
   int singular = 0;
-  bool dom = true, swaps = false;
-  double rho_line = 0.0;  // largest (|DL| + |DU|) / |D| of the line's rows
+  bool swaps = false;
   double Dc = 0.0, DUc = 0.0;
   // row factors PF rows ahead
   constexpr int PF = 8;
@@ -122,10 +220,6 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
         DLn = -((th)*LeftFac);
         Dn = 1.0 + (th)*CenterFac - (th)*RightFac;
       }
-      // L, R >= 0 and finite, theta >= 0: every row has D >= 1 + |DL| + |DU|
-      // in exact arithmetic (false for NaN too)
-      dom = dom && LeftFac >= 0.0 && RightFac >= 0.0 && LeftFac <= DBL_MAX && RightFac <= DBL_MAX && th >= 0.0;
-      rho_line = fmax(rho_line, (fabs(DLn) + fabs(DUn)) / fabs(Dn));
       if (l == 1) {
         Dc = Dn;
         DUc = DUn;
@@ -169,33 +263,7 @@ __global__ __launch_bounds__(kBlock) void k_line_lu(DiffArgs A, double *lu, uint
   if (Dc == 0.0 && !singular) singular = n;
   fD[base + sL * (long long)(rmin + n)] = Dc;
   sing[gid] = singular;
-  if (!dom) atomicAdd(ndom, 1);
-  if (swaps) atomicAdd(ndom + 1, 1);
-  // the sweep's largest row ratio (non-negative doubles order as their bit
-  // patterns); lines that are not dominant count as 1
-  const double r = (dom && rho_line < 1.0) ? rho_line : 1.0;
-  if (rho) atomicMax(rho, (unsigned long long)__double_as_longlong(r));
-  // the Jacobi sweeps the line needs (0: more than kJacobiMaxSweepsX); the
-  // number of lines that need at most that many and the largest ratio
-  // among them
-  if (jl) {
-    const int sw = dom ? jacobi_sweeps_needed(r, kJacobiMaxSweepsX) : 0;
-    jl[gid] = (uint8_t)sw;
-    if (sw > 0) {
-      atomicMax(rho_j, (unsigned long long)__double_as_longlong(r));
-      atomicAdd(njl, 1);
-    }
-  }
-}
-
-// the counts and ratios that k_line_lu accumulates
-__global__ void k_zero_counts(int *ndom, unsigned long long *rho, unsigned long long *rho_j, int *njl) {
-  ndom[0] = ndom[1] = 0;
-  if (rho) *rho = 0ull;
-  if (rho_j) {
-    *rho_j = 0ull;
-    *njl = 0;
-  }
+  if (swaps) atomicAdd(&cnt->nswap, 1);
 }
 
 // theta-scheme line solve.  Row l (cell c = rmin-1+l) of the system
@@ -607,7 +675,7 @@ __global__ __launch_bounds__(kBlock) void k_cn_jacobi(DiffArgs A) {
 // stores stay coalesced: a bin's q is read row block by row block (lane l
 // of block m: row 64 M w + 64 m + l) and turned into the lane's rows
 // through LDS, the solution the same way back.  The row factors L, R are
-// formed from kappa, sigma_nx and kx as k_line_lr forms them (same
+// formed from kappa, sigma_nx and kx as k_line_rows forms them (same
 // arithmetic, so the same values as the factor cache) once per line, with
 // the Jacobi coefficients; then every aloft bin of the line in turn: its
 // right-hand side as k_cn_jacobi forms it (the next bin's q already in
@@ -1130,33 +1198,36 @@ hipError_t launch_cn_nb(hipStream_t s, const DiffArgs &a) {
 
 }  // namespace
 
-hipError_t launch_line_lr(hipStream_t s, const DiffArgs &a, double *lr) {
-  const long long cells = (long long)a.g.Na * a.g.N * a.g.Nb;
-  dim3 grid((unsigned)((cells + kBlock - 1) / kBlock));
+namespace {
+
+template <int W>
+void launch_line_rows_w(hipStream_t s, const DiffArgs &a, double *lr, const LineStats &st, dim3 grid) {
   switch (a.g.dir) {
-    case 0: hipLaunchKernelGGL((k_line_lr<0>), grid, dim3(kBlock), 0, s, a, lr); break;
-    case 1: hipLaunchKernelGGL((k_line_lr<1>), grid, dim3(kBlock), 0, s, a, lr); break;
-    default: hipLaunchKernelGGL((k_line_lr<2>), grid, dim3(kBlock), 0, s, a, lr); break;
+    case 0: hipLaunchKernelGGL((k_line_rows<0, W>), grid, dim3(64 * W), 0, s, a, lr, st); break;
+    case 1: hipLaunchKernelGGL((k_line_rows<1, W>), grid, dim3(64 * W), 0, s, a, lr, st); break;
+    default: hipLaunchKernelGGL((k_line_rows<2, W>), grid, dim3(64 * W), 0, s, a, lr, st); break;
   }
+}
+
+}  // namespace
+
+hipError_t launch_line_rows(hipStream_t s, const DiffArgs &a, double *lr, const LineStats &st) {
+  const long long lines = (long long)a.g.Na * a.g.Nb;
+  const dim3 grid((unsigned)((lines + 63) / 64));
+  // (runs of 8 to 16 rows and more: at 240 and 360 rows 16 waves take 63 us, 8 take 66)
+  if (a.g.N >= 128) launch_line_rows_w<16>(s, a, lr, st, grid);
+  else launch_line_rows_w<8>(s, a, lr, st, grid);
   return hipGetLastError();
 }
 
-hipError_t launch_line_lu(hipStream_t s, const DiffArgs &a, double *lu, uint8_t *piv, int *sing, int *ndom,
-                          unsigned long long *rho, uint8_t *jl, unsigned long long *rho_j, int *njl) {
-  if ((jl == nullptr) != (rho_j == nullptr) || (jl == nullptr) != (njl == nullptr)) return hipErrorInvalidValue;
+hipError_t launch_line_lu(hipStream_t s, const DiffArgs &a, double *lu, uint8_t *piv, int *sing, LineCounts *cnt,
+                          bool gated) {
   const long long lines = (long long)a.g.Na * a.g.Nb;
   dim3 grid((unsigned)((lines + kBlock - 1) / kBlock));
-  hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(1), 0, s, ndom, rho, rho_j, njl);
   switch (a.g.dir) {
-    case 0:
-      hipLaunchKernelGGL((k_line_lu<0>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, ndom, rho, jl, rho_j, njl);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_line_lu<1>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, ndom, rho, jl, rho_j, njl);
-      break;
-    default:
-      hipLaunchKernelGGL((k_line_lu<2>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, ndom, rho, jl, rho_j, njl);
-      break;
+    case 0: hipLaunchKernelGGL((k_line_lu<0>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, cnt, gated); break;
+    case 1: hipLaunchKernelGGL((k_line_lu<1>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, cnt, gated); break;
+    default: hipLaunchKernelGGL((k_line_lu<2>), grid, dim3(kBlock), 0, s, a, lu, piv, sing, cnt, gated); break;
   }
   return hipGetLastError();
 }
