@@ -108,7 +108,8 @@ int ash3d_tr_create(const ash3d_tr_desc *desc, ash3d_tr_ctx **ctx);
 int ash3d_tr_destroy(ash3d_tr_ctx *ctx);
 
 /* Host <-> device copies of the array groups in mask (ASH3D_SYNC_*).
- * sync_to_host blocks until the data is on the host. */
+ * sync_to_host blocks until the data is on the host; for large states a few
+ * threads of its own write the ts1 level there while ts0 is copied. */
 int ash3d_tr_sync_from_host(ash3d_tr_ctx *ctx, uint32_t mask);
 int ash3d_tr_sync_to_host(ash3d_tr_ctx *ctx, uint32_t mask);
 /* Wait for all queued work of the context. */

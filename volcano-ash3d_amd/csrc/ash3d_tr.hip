@@ -141,6 +141,7 @@ struct ash3d_tr_ctx {
   int *swap_h = nullptr;
   hipEvent_t ndom_ev[3] = {}, swap_ev[3] = {};
   int ndom_state[3] = {0, 0, 0}, swap_state[3] = {0, 0, 0};
+  hipEvent_t rb_ev[kReadbackEvents] = {};
   bool capturing = false;
   // the velocity ghosts hold Set_BC(1)'s values for the current interior
   // velocities (cleared by every entry point that writes velocities)
@@ -1100,6 +1101,8 @@ int ash3d_tr_destroy(ash3d_tr_ctx *x) {
     if (x->ndom_ev[k]) hipEventDestroy(x->ndom_ev[k]);
     if (x->swap_ev[k]) hipEventDestroy(x->swap_ev[k]);
   }
+  for (auto &e : x->rb_ev)
+    if (e) hipEventDestroy(e);
   for (auto &e : x->ev_pool) {
     hipEventDestroy(e.first);
     hipEventDestroy(e.second);
@@ -1168,14 +1171,15 @@ int ash3d_tr_sync_to_host(ash3d_tr_ctx *x, uint32_t mask) {
   const ash3d_tr_desc &h = x->host;
   const Dims &d = x->d;
   if (mask & ASH3D_SYNC_CONCEN) {
-    // materialise ts1; the recorded state stays valid (ts1 now holds
-    // exactly what the record says), so captured steps may still follow
-    if (x->ts1_state == TS1_MIRROR) {
-      HIPCHK(launch_mirror_interior(x->stream, d, x->ts0(), x->ts1()));
-    } else if (x->ts1_state == TS1_ZERO) {
-      HIPCHK(launch_fill(x->stream, x->ts1(), x->n_conc(), 0.0));
+    // the ts1 level as recorded (the record stays valid, so captured steps
+    // may still follow)
+    if (x->ts1_state == TS1_EXPLICIT) {
+      if ((rc = download(x, h.concen_pd, x->c, 2 * x->n_conc()))) return rc;
+    } else if (h.concen_pd) {
+      for (auto &e : x->rb_ev)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      HIPCHK(download_levels(x->stream, d, x->ts1_state == TS1_ZERO, x->ts0(), x->ts1(), h.concen_pd, x->rb_ev));
     }
-    if ((rc = download(x, h.concen_pd, x->c, 2 * x->n_conc()))) return rc;
   }
   if (mask & ASH3D_SYNC_WINDS) {
     if ((rc = download(x, h.vx_pd, x->vx, d.ncell)) || (rc = download(x, h.vy_pd, x->vy, d.ncell)) ||

@@ -244,13 +244,14 @@ __global__ __launch_bounds__(kBlock) void k_fill(double *p, long long n, double 
   for (long long q = t; q < n; q += stride) p[q] = v;
 }
 
-// ts1 = interior(ts0), zero ghosts: the content the reference leaves in ts1
+// ts1 = interior(ts0), zero ghosts, on x rows [r0, r1): the content the reference leaves in ts1
 // after any sweep (zero fill, interior rows written, copied to ts0).
-__global__ __launch_bounds__(kBlock) void k_mirror(Dims d, const double *c0, double *c1) {
+__global__ __launch_bounds__(kBlock) void k_mirror(Dims d, const double *c0, double *c1, long long r0,
+                                                  long long r1) {
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-  const long long tot = d.ncell * d.ns;
+  const long long tot = r1 * d.sy;
   const long long stride = (long long)gridDim.x * kBlock;
-  for (long long q = t; q < tot; q += stride) {
+  for (long long q = r0 * d.sy + t; q < tot; q += stride) {
     const long long cell = q % d.ncell;
     const int i = (int)(cell % d.sy) - 1;
     const int j = (int)((cell / d.sy) % (d.ny + 4)) - 1;
@@ -382,10 +383,12 @@ hipError_t launch_fill(hipStream_t s, double *p, long long n, double v) {
   return hipGetLastError();
 }
 
-hipError_t launch_mirror_interior(hipStream_t s, const Dims &d, const double *c0, double *c1) {
-  unsigned b = blocks_for(d.ncell * d.ns);
+hipError_t launch_mirror_interior(hipStream_t s, const Dims &d, const double *c0, double *c1, long long r0,
+                                  long long r1) {
+  if (r1 <= r0) return hipSuccess;
+  unsigned b = blocks_for((r1 - r0) * d.sy);
   if (b > 8192) b = 8192;
-  hipLaunchKernelGGL(k_mirror, dim3(b), dim3(kBlock), 0, s, d, c0, c1);
+  hipLaunchKernelGGL(k_mirror, dim3(b), dim3(kBlock), 0, s, d, c0, c1, r0, r1);
   return hipGetLastError();
 }
 

@@ -243,7 +243,15 @@ hipError_t launch_zero_ghosts(hipStream_t s, const Dims &d, double *c0);
 // dst's ghost cells (every bin) = src's
 hipError_t launch_copy_ghosts(hipStream_t s, const Dims &d, const double *src, double *dst);
 hipError_t launch_fill(hipStream_t s, double *p, long long n, double v);
-hipError_t launch_mirror_interior(hipStream_t s, const Dims &d, const double *c0, double *c1);
+// x rows [r0, r1) of all levels of all bins
+hipError_t launch_mirror_interior(hipStream_t s, const Dims &d, const double *c0, double *c1, long long r0,
+                                  long long r1);
+// both levels of the state into host (2 * ncell * ns doubles) where the ts1
+// level is ts0's interior with zero ghosts (or zero); c1 is scratch.  Waits
+// for the copies (host_state.hip)
+constexpr int kReadbackEvents = 4;
+hipError_t download_levels(hipStream_t s, const Dims &d, bool zero, const double *c0, double *c1, double *host,
+                           hipEvent_t *ev);
 // umbrella source: 3x3 patch averaging (levels ibase..itop) and insertion
 // (levels 1..nz+1) for bins < ngs; umbrella winds added to vx, vy
 hipError_t launch_umbrella_source(hipStream_t s, const Dims &d, double *c0, int iv, int jv, double dt, int ibase,
