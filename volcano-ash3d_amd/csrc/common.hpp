@@ -332,7 +332,11 @@ hipError_t launch_line_rows(hipStream_t s, const DiffArgs &a, double *lr, const 
 struct PartLayout {
   long long st0, sta, stb, str;
   long long lr0, lra, lrb, lrr, lr_ncell;
-  const double *kap = nullptr;  // cell volumes in the state's layout (adjoint only)
+  const double *kap = nullptr;  // cell volumes in the state's layout (x lines, adjoint)
+  // x lines (str == 1), which form the row factors themselves: sigma_nx in
+  // the state's layout and kx, cell i of line (a, b) at kk[ka*a + kb*b + i]
+  const double *sig = nullptr, *kk = nullptr;
+  long long ka = 0, kb = 0;
 };
 // adjoint: lambda <- K B A^{-1} K^{-1} lambda (= B^T A^{-T} lambda, since
 // kappa_l R_l = kappa_{l+1} L_{l+1} makes K A and K B symmetric, K = diag kappa)
