@@ -149,10 +149,13 @@ struct ash3d_tr_ctx {
   // the glue's zeroing of the ts0 ghosts, not yet launched: the next
   // transport step's Set_BC(1) rewrites every concentration ghost from
   // interior cells, so it stands in for it; every other entry point but
-  // the met/wind updates launches it first (the vent-column source too: it
-  // adds into the ghost cell above the column, which a later reader must
-  // see as zero plus the source)
+  // the met/wind updates and the vent-column source launches it first (the
+  // source adds into the ghost cell above the column, which a later reader
+  // must see as zero plus the source: it writes that, see src_i)
   bool ghost_zero_pending = false;
+  // while that zeroing is pending: the column whose ghost cell above the top
+  // layer already holds zero plus a source (0: none), left out of it
+  int src_i = 0, src_j = 0;
   // umbrella source: device copies of the stencil + patch flux and of the
   // two wind planes, uploaded through one pinned staging buffer each
   double *umb_src = nullptr, *umb_wind = nullptr;
@@ -169,11 +172,21 @@ struct ash3d_tr_ctx {
   bool lu_args_full[3] = {false, false, false};  // the dgtsv-order solves may read the factors
   DiffArgs graph_lu[2][3] = {};
   bool graph_lu_on[2][3] = {}, graph_lu_full[2][3] = {};
+  // sweeps captured without the dgtsv-order alternative, every line being
+  // dominant (cap_dom: in the capture under way), and the row factors
+  // (ln_stamp) for which that was seen; the step's own arguments, for an
+  // eager step in place of a replay when it no longer holds
+  bool cap_dom[3] = {}, graph_dom[2][3] = {};
+  long long ln_stamp[3] = {0, 0, 0}, graph_stamp[2][3] = {};
+  struct StepArgs {
+    double dt, imp_fac;
+    int32_t use_diffusion, use_cn;
+    std::vector<int32_t> aloft;
+  } graph_step[2];
   bool graph_tgeom[2] = {false, false};  // the graph reads the transposed geometry
   long long fac_groups = 0;
-  double *flux = nullptr;  // source column staging (nz+1)*ns
   // pinned host ring for the source columns: the caller's buffer is copied
-  // into a slot, so the upload is asynchronous and the host may run ahead
+  // into a slot, which the kernel reads, so the host may run ahead
   static constexpr int kFluxRing = 4;
   double *flux_pinned[kFluxRing] = {};
   hipEvent_t flux_ev[kFluxRing] = {};
@@ -287,7 +300,7 @@ int check_ctx(ash3d_tr_ctx *x) {
   if (rc) return rc;
   if (x->ghost_zero_pending) {
     x->ghost_zero_pending = false;
-    HIPCHK(launch_zero_ghosts(x->stream, x->d, x->ts0()));
+    HIPCHK(launch_zero_ghosts(x->stream, x->d, x->ts0(), x->src_i, x->src_j));
   }
   return 0;
 }
@@ -340,11 +353,11 @@ int set_bc1(ash3d_tr_ctx *x, bool velocities, double *state = nullptr, bool conc
   ProfScope ps(x, ASH3D_PROF_BC);
   // Set_BC(1) on velocities is a projection (every ghost a copy of an
   // interior or wrapped cell that the pass does not write), so it is
-  // skipped while the ghosts already hold its values; a captured graph
-  // always contains it
-  if (velocities && (x->capturing || !x->vel_bc_ok))
+  // skipped while the ghosts already hold its values (a captured step runs
+  // it before the capture, and before a replay when velocities changed)
+  if (velocities && !x->vel_bc_ok)
     HIPCHK(launch_set_bc1_vel(x->stream, x->d, x->periodic, x->vx, x->vy, x->vz, x->vf));
-  if (velocities && !x->capturing) x->vel_bc_ok = true;
+  if (velocities) x->vel_bc_ok = true;
   if (conc) HIPCHK(launch_set_bc1_conc(x->stream, x->d, x->periodic, state ? state : x->ts0()));
   return 0;
 }
@@ -528,6 +541,7 @@ int run_line_rows(ash3d_tr_ctx *x, int dir, const DiffArgs &a) {
   x->ln_rmax[dir] = a.g.rmax;
   x->lu_state[dir] = ash3d_tr_ctx::LU_NONE;
   x->swap_state[dir] = 0;
+  ++x->ln_stamp[dir];
   return 0;
 }
 
@@ -735,7 +749,7 @@ int try_cn_partitioned(ash3d_tr_ctx *x, int dir, DiffArgs &a, int *rc, bool adjo
   // partitioned solves take the lines the forward's took, so that the
   // sweeps the forward ran as Jacobi sweeps get their transpose)
   if (dgtsv_sweep(x, dir, n)) return 0;
-  const int hn = host_ndom(x, dir);
+  const int hn = x->capturing && x->cap_dom[dir] ? 0 : host_ndom(x, dir);
   if (hn > 0) return 0;
   const PartLayout lay = part_layout(x, dir, a);
   a.sel = 1;
@@ -1048,7 +1062,7 @@ int ash3d_tr_create(const ash3d_tr_desc *desc, ash3d_tr_ctx **out) {
       (rc = dev_alloc(&x->ofxz1, x->n_xz())) || (rc = dev_alloc(&x->ofxz2, x->n_xz())) ||
       (rc = dev_alloc(&x->ofyz1, x->n_yz())) || (rc = dev_alloc(&x->ofyz2, x->n_yz())) ||
       (rc = dev_alloc(&x->ofxy1, x->n_xy())) || (rc = dev_alloc(&x->ofxy2, x->n_xy())) ||
-      (rc = dev_alloc(&x->dep, x->n_dep())) || (rc = dev_alloc(&x->flux, (long long)(d.nz + 1) * d.ns))) {
+      (rc = dev_alloc(&x->dep, x->n_dep()))) {
     std::string msg = g_err;
     ash3d_tr_destroy(x);
     g_err = msg;
@@ -1080,7 +1094,7 @@ int ash3d_tr_destroy(ash3d_tr_ctx *x) {
   if (x->stream) hipStreamSynchronize(x->stream);
   double *ptrs[] = {x->c, x->vx, x->vy, x->vz, x->vh, x->vf, x->kap, x->sx, x->sy, x->sz, x->kx, x->ky, x->kz,
                     x->ddx, x->ddy, x->ofxz1, x->ofxz2, x->ofyz1, x->ofyz2, x->ofxy1, x->ofxy2, x->dep,
-                    x->fac, x->flux, x->tot, x->tq, x->tkap, x->tsx, x->tkx, x->lam, x->snap_b,
+                    x->fac, x->tot, x->tq, x->tkap, x->tsx, x->tkx, x->lam, x->snap_b,
                     x->snap_z, x->adj_sb, x->sink, x->src_grad, x->col, x->lr[0], x->lr[1], x->lr[2],
                     x->lu[0], x->lu[1], x->lu[2], x->ln[0], x->ln[1], x->ln[2], x->junk, x->prod, x->dtvc};
   for (double *p : ptrs)
@@ -1429,6 +1443,7 @@ int ash3d_tr_step_glue(ash3d_tr_ctx *x) {
   ProfScope ps(x, ASH3D_PROF_GLUE);
   if (x->ts1_state == TS1_MIRROR) {
     x->ghost_zero_pending = true;  // launched by the next entry point unless a step comes first
+    x->src_i = x->src_j = 0;
   } else if (x->ts1_state == TS1_ZERO) {
     HIPCHK(launch_fill(x->stream, x->ts0(), x->n_conc(), 0.0));
   } else {
@@ -1440,24 +1455,32 @@ int ash3d_tr_step_glue(ash3d_tr_ctx *x) {
 }
 
 int ash3d_tr_source_column_add(ash3d_tr_ctx *x, int32_t ivent, int32_t jvent, double dt, const double *flux) {
-  int rc = check_ctx(x);
+  int rc = check_ctx_keep(x);
   if (rc) return rc;
   if (!flux) return fail(ASH3D_TR_EINVAL, "null flux");
   if (ivent < 1 || ivent > x->d.nx || jvent < 1 || jvent > x->d.ny)
     return fail(ASH3D_TR_EINVAL, "vent (%d,%d) outside the grid", ivent, jvent);
+  // the glue's pending zeroing stays pending: of the ghosts it would zero,
+  // the source reads only the cell above the top layer of its column, as
+  // zero (a second column before the step has the zeroing launched)
+  const bool seen = x->src_i == ivent && x->src_j == jvent;
+  if (x->ghost_zero_pending && x->src_i != 0 && !seen && (rc = check_ctx(x))) return rc;
+  const bool top_zero = x->ghost_zero_pending && !seen;
   const size_t bytes = sizeof(double) * (size_t)(x->d.nz + 1) * x->d.ns;
   const int k = x->flux_slot;
   if (!x->flux_pinned[k]) {
     HIPCHK(hipHostMalloc((void **)&x->flux_pinned[k], bytes, hipHostMallocDefault));
     HIPCHK(hipEventCreateWithFlags(&x->flux_ev[k], hipEventDisableTiming));
   }
-  if (x->flux_used[k]) HIPCHK(hipEventSynchronize(x->flux_ev[k]));  // its last upload has been read
+  if (x->flux_used[k]) HIPCHK(hipEventSynchronize(x->flux_ev[k]));  // its last column has been added
   std::memcpy(x->flux_pinned[k], flux, bytes);
-  HIPCHK(hipMemcpyAsync(x->flux, x->flux_pinned[k], bytes, hipMemcpyHostToDevice, x->stream));
+  // (the kernel reads the pinned column itself: a few KB over the link, in
+  // place of a copy of its own before it)
+  HIPCHK(launch_source_add(x->stream, x->d, x->ts0(), ivent, jvent, dt, x->flux_pinned[k], top_zero));
   HIPCHK(hipEventRecord(x->flux_ev[k], x->stream));
+  if (top_zero) { x->src_i = ivent; x->src_j = jvent; }
   x->flux_used[k] = true;
   x->flux_slot = (k + 1) % ash3d_tr_ctx::kFluxRing;
-  HIPCHK(launch_source_add(x->stream, x->d, x->ts0(), ivent, jvent, dt, x->flux));
   return 0;
 }
 
@@ -2012,9 +2035,28 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     HIPCHK(hipGraphExecDestroy(x->graph[slot]));
     x->graph[slot] = nullptr;
   }
-  for (int k = 0; k < 3; ++k) x->lu_args_set[k] = false;
+  for (int k = 0; k < 3; ++k) x->cap_dom[k] = false;
   x->graph_dtv[slot] = -1.0;
   if (use_diffusion && x->adv_fused && (rc = ensure_dtv(x, dt))) return rc;  // (outside the capture)
+  // (outside the capture too) the velocity ghosts, the line factors, and
+  // which sweeps need no dgtsv-order alternative
+  if ((rc = set_bc1(x, true, nullptr, false))) return rc;
+  if (use_diffusion && use_cn) {
+    int32_t b[6];
+    full_bounds(x, b);
+    for (int dir = 0; dir < 3; ++dir) {
+      DiffArgs a = diff_args(x, dir, dt, imp_fac, is_aloft, b);
+      if (dir == 0) transpose_x_args(x, b, a);
+      const int n = a.g.rmax - a.g.rmin + 1;
+      if (n <= 1) continue;
+      const bool full = dgtsv_sweep(x, dir, n);
+      if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, full))) return rc;
+      x->cap_dom[dir] = !full && x->cnt_h;
+    }
+    HIPCHK(hipStreamSynchronize(x->stream));
+    for (int dir = 0; dir < 3; ++dir) x->cap_dom[dir] = x->cap_dom[dir] && x->cnt_h[dir].ndom == 0;
+  }
+  for (int k = 0; k < 3; ++k) x->lu_args_set[k] = false;
   HIPCHK(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
   x->capturing = true;
   int rc2 = ash3d_tr_step_glue(x);
@@ -2034,8 +2076,12 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     x->graph_lu_on[slot][k] = x->lu_args_set[k];
     x->graph_lu[slot][k] = x->lu_args[k];
     x->graph_lu_full[slot][k] = x->lu_args_full[k];
+    x->graph_dom[slot][k] = x->cap_dom[k];
+    x->graph_stamp[slot][k] = x->ln_stamp[k];
   }
   x->graph_tgeom[slot] = use_diffusion && use_cn;
+  x->graph_step[slot] = {dt, imp_fac, use_diffusion, use_cn,
+                         is_aloft ? std::vector<int32_t>(is_aloft, is_aloft + x->d.ns) : std::vector<int32_t>()};
   return 0;
 }
 
@@ -2054,6 +2100,20 @@ int ash3d_tr_graph_launch(ash3d_tr_ctx *x, int32_t itime) {
     if (!x->graph_lu_on[slot][k]) continue;
     DiffArgs a = x->graph_lu[slot][k];
     if ((rc = ensure_lr(x, k, a)) || (rc = ensure_lu(x, k, a, x->graph_lu_full[slot][k]))) return rc;
+  }
+  if ((rc = set_bc1(x, true, nullptr, false))) return rc;
+  // new factors since the lines were seen to be dominant: wait for their
+  // counts; a step with other lines is launched as it is
+  for (int k = 0; k < 3; ++k) {
+    if (!x->graph_dom[slot][k] || x->graph_stamp[slot][k] == x->ln_stamp[k]) continue;
+    HIPCHK(hipStreamSynchronize(x->stream));
+    if (x->cnt_h[k].ndom != 0) {
+      const auto &st = x->graph_step[slot];
+      if ((rc = ash3d_tr_step_glue(x))) return rc;
+      return ash3d_tr_step(x, itime, st.dt, st.use_diffusion, st.use_cn, st.imp_fac,
+                           st.aloft.empty() ? nullptr : st.aloft.data());
+    }
+    x->graph_stamp[slot][k] = x->ln_stamp[k];
   }
   HIPCHK(hipGraphLaunch(x->graph[slot], x->stream));
   x->ts1_state = TS1_MIRROR;
@@ -2205,10 +2265,11 @@ int ash3d_tr_minmax_index(ash3d_tr_ctx *x, int32_t ivent, int32_t jvent, int32_t
 int ash3d_tr_step_subgrid(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t use_diffusion, int32_t use_cn,
                           double imp_fac, const int32_t *is_aloft, int32_t ivent, int32_t jvent, int32_t kvent,
                           double thresh, int32_t bounds[6]) {
-  int rc = check_ctx(x);
+  int rc = check_ctx_keep(x);
   if (rc) return rc;
   int32_t b[6];
   if ((rc = set_bc1(x, true))) return rc;  // src/Ash3d.F90:491
+  x->ghost_zero_pending = false;  // (every ts0 ghost rewritten)
   if ((rc = minmax_index(x, ivent, jvent, kvent, thresh, b))) return rc;
   if (bounds)
     for (int q = 0; q < 6; ++q) bounds[q] = b[q];

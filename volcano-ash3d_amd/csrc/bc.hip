@@ -61,7 +61,7 @@ enum { GH_ZERO = 0, GH_BC1 = 1, GH_BC2 = 2, GH_COPY = 3 };
 // sequential x (periodic override), y, z mirrors leave every ghost equal to
 // c(xmap(i), clamp(j), clamp(k)).
 __global__ __launch_bounds__(kBlock) void k_ghosts_all(Dims d, int periodic, int mode, double *c0,
-                                                      const double *src) {
+                                                      const double *src, int ki, int kj) {
   const int n = (int)blockIdx.y;
   long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   const long long plane = (long long)(d.nx + 4) * (d.ny + 4);
@@ -78,6 +78,7 @@ __global__ __launch_bounds__(kBlock) void k_ghosts_all(Dims d, int periodic, int
     t %= ring;
   }
   if (!ghost_cell(d, k, t, i, j)) return;
+  if (k == d.nz + 1 && i == ki && j == kj) return;  // (the ghost cell of a source column)
   double *c = c0 + d.ncell * n;
   double v = 0.0;
   if (mode == GH_BC1) {
@@ -92,12 +93,12 @@ __global__ __launch_bounds__(kBlock) void k_ghosts_all(Dims d, int periodic, int
 }
 
 hipError_t launch_ghosts(hipStream_t s, const Dims &d, int periodic, int mode, double *c0,
-                         const double *src = nullptr) {
+                         const double *src = nullptr, int ki = -9, int kj = -9) {
   const long long plane = (long long)(d.nx + 4) * (d.ny + 4);
   const long long ring = 4LL * (d.nx + 4) + 4LL * d.ny;
   const long long per_bin = 4 * plane + (long long)d.nz * ring;
   dim3 grid((unsigned)((per_bin + kBlock - 1) / kBlock), d.ns);
-  hipLaunchKernelGGL(k_ghosts_all, grid, dim3(kBlock), 0, s, d, periodic, mode, c0, src);
+  hipLaunchKernelGGL(k_ghosts_all, grid, dim3(kBlock), 0, s, d, periodic, mode, c0, src, ki, kj);
   return hipGetLastError();
 }
 
@@ -261,15 +262,16 @@ __global__ __launch_bounds__(kBlock) void k_mirror(Dims d, const double *c0, dou
   }
 }
 
-// concen(iv,jv,k,n,ts0) += dt*flux(k,n), k = 1..nz+1 (src/Ash3d.F90:428-431)
+// concen(iv,jv,k,n,ts0) += dt*flux(k,n), k = 1..nz+1 (src/Ash3d.F90:428-431);
+// top_zero: the ghost cell k = nz+1 counts as zero (its zeroing is pending)
 __global__ __launch_bounds__(kBlock) void k_source(Dims d, double *c0, int iv, int jv, double dt,
-                                                  const double *flux) {
+                                                  const double *flux, bool top_zero) {
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   const long long tot = (long long)(d.nz + 1) * d.ns;
   if (t >= tot) return;
   const int k = (int)(t % (d.nz + 1)) + 1, n = (int)(t / (d.nz + 1));
   const long long o = d.p3(iv, jv, k) + d.ncell * n;
-  c0[o] = c0[o] + dt * flux[t];
+  c0[o] = (top_zero && k == d.nz + 1 ? 0.0 : c0[o]) + dt * flux[t];
 }
 
 // Umbrella source (src/Ash3d.F90:447-460), one thread per (level k =
@@ -350,8 +352,8 @@ hipError_t launch_set_bc2_face(hipStream_t s, const Dims &d, int periodic, int d
   return hipGetLastError();
 }
 
-hipError_t launch_zero_ghosts(hipStream_t s, const Dims &d, double *c0) {
-  return launch_ghosts(s, d, 0, GH_ZERO, c0);
+hipError_t launch_zero_ghosts(hipStream_t s, const Dims &d, double *c0, int keep_i, int keep_j) {
+  return launch_ghosts(s, d, 0, GH_ZERO, c0, nullptr, keep_i > 0 ? keep_i : -9, keep_j > 0 ? keep_j : -9);
 }
 
 hipError_t launch_copy_ghosts(hipStream_t s, const Dims &d, const double *src, double *dst) {
@@ -410,9 +412,9 @@ hipError_t launch_umbrella_winds(hipStream_t s, const Dims &d, double *vx, doubl
 }
 
 hipError_t launch_source_add(hipStream_t s, const Dims &d, double *c0, int iv, int jv, double dt,
-                             const double *flux) {
+                             const double *flux, bool top_zero) {
   const long long tot = (long long)(d.nz + 1) * d.ns;
-  hipLaunchKernelGGL(k_source, dim3(blocks_for(tot)), dim3(kBlock), 0, s, d, c0, iv, jv, dt, flux);
+  hipLaunchKernelGGL(k_source, dim3(blocks_for(tot)), dim3(kBlock), 0, s, d, c0, iv, jv, dt, flux, top_zero);
   return hipGetLastError();
 }
 

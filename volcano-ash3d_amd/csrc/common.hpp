@@ -239,7 +239,8 @@ hipError_t launch_set_bc2(hipStream_t s, const Dims &d, int periodic, double *c0
 // Set_BC(2) on the dir (0: x, 1: y) ghosts of the interior rows only
 hipError_t launch_set_bc2_face(hipStream_t s, const Dims &d, int periodic, int dir, double *c0);
 hipError_t launch_neumann_dir(hipStream_t s, const Dims &d, int dir, int periodic, double *c0);
-hipError_t launch_zero_ghosts(hipStream_t s, const Dims &d, double *c0);
+// (keep_i, keep_j > 0: not the cell (keep_i, keep_j, nz+1))
+hipError_t launch_zero_ghosts(hipStream_t s, const Dims &d, double *c0, int keep_i = 0, int keep_j = 0);
 // dst's ghost cells (every bin) = src's
 hipError_t launch_copy_ghosts(hipStream_t s, const Dims &d, const double *src, double *dst);
 hipError_t launch_fill(hipStream_t s, double *p, long long n, double v);
@@ -258,8 +259,9 @@ hipError_t launch_umbrella_source(hipStream_t s, const Dims &d, double *c0, int 
                                   int itop, int ngs, const double *st, const double *fu);
 hipError_t launch_umbrella_winds(hipStream_t s, const Dims &d, double *vx, double *vy, int ibase, int itop,
                                  const double *uvx, const double *uvy);
+// top_zero: the ghost cell above the column counts as zero
 hipError_t launch_source_add(hipStream_t s, const Dims &d, double *c0, int iv, int jv, double dt,
-                             const double *flux);
+                             const double *flux, bool top_zero);
 hipError_t launch_advect(hipStream_t s, const AdvArgs &a, int nb);
 
 // the launch launch_advect(s, a, nb) would issue
