@@ -64,3 +64,17 @@ def test_captured_steps(pkg, oracle, tr):  # noqa: F811
     assert_same(E.st, G.st)
     E.close()
     G.close()
+
+
+@pytest.mark.parametrize("n", [2, 8, 9, 56, 57, 63, 64, 65, 72, 73, 79, 80, 81])
+@pytest.mark.parametrize("ns", [1, 2, 5])
+def test_kept_right_hand_sides(pkg, oracle, tr, n, ns):  # noqa: F811
+    """Lines whose eliminated right-hand sides stay in registers (up to 64
+    and up to 80 cells) and longer ones; a box inside longer lines."""
+    for shape, box in (((9, n, 4), None), ((7, 5, n), None), ((5, 90, 85), (1, 5, 4, 3 + n, 2, 1 + n))):
+        st = pkg.workloads.random_state(*shape, ns, seed=n + ns, latlon=True)
+        if box:
+            st.bounds = box
+        st.dt *= 30.0
+        a, b = run_both(pkg, oracle, tr, st, [("diffCN_y",), ("diffCN_z",)] * 3)
+        assert_same(a, b)

@@ -10,11 +10,15 @@
 // sides) is in flight in registers while the one before is worked on.  x
 // lines are contiguous in memory: a wave turns their chunks into its lanes'
 // lines through LDS on the way in and out.  The eliminated right-hand sides
-// wait in the ts1 slot (on larger states their traffic, half of the sweep's,
-// is what bounds it: 360x240x50x15 y 653 -> 621, z 529 -> 489 us).  Against one thread per line and 2 or 8 bins
-// (k_diff_cn, k_diff_cn_xrows, which keep the sweeps with row interchanges):
-// 240x160x50x8 x, y, z 380, 347, 145 us -> 161, 138, 110 us.  The arithmetic
-// is dgtsv's, so the results are the same bits.
+// wait in registers on lines of up to 80 cells (two registers a row), on
+// longer ones in the ts1 slot, whose traffic is then half of the sweep's and,
+// on larger states, what bounds it (y at 240x160x50x8: 569 MB in 148 us, 3.9
+// TB/s).  Against one thread per line and 2 or 8 bins (k_diff_cn,
+// k_diff_cn_xrows, which keep the sweeps with row interchanges): 240x160x50x8
+// x, y, z 380, 347, 145 us -> 175, 148, 78 (z with the ts1 slot 118).
+// Quotients from inverses (fewer dependent operations) and two chunks in
+// flight gained nothing.  The arithmetic is dgtsv's, so the results are the
+// same bits.
 #include <algorithm>
 
 #include "common.hpp"
@@ -42,8 +46,11 @@ __device__ __forceinline__ void wg_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <bool XR, int NW, int RC>
-__global__ __launch_bounds__(64 * NW) void k_cn_exact(ExactArgs E) {
+// KC > 0: the eliminated right-hand sides of up to KC chunks stay in
+// registers instead of the scratch.
+template <bool XR, int NW, int RC, int KC>
+__global__ __launch_bounds__(64 * NW, (KC == 8 && NW == 4) ? 3 : 1) void k_cn_exact(ExactArgs E) {
+  static_assert(!XR || KC == 0, "");
   constexpr int RPW = RC / NW;  // rows of a chunk that each wave loads
   static_assert(RC % NW == 0, "");
   const DiffArgs &A = E.A;
@@ -137,43 +144,51 @@ __global__ __launch_bounds__(64 * NW) void k_cn_exact(ExactArgs E) {
   load_q(0);
   put_f(0);
   wg_lds_barrier();
-  for (int k = 0; k < nch; ++k) {
-    double q[RC];
-    take_q(q);
-    if (k + 1 < nch) {
-      load_f(k + 1);
-      load_q(k + 1);
-    }
-    const double(*s)[RC][64] = s_f[k & 1];
-    if (on) {
+  double Y[KC > 0 ? KC * RC : 1];
+  constexpr int kUnroll = KC > 0 ? KC : 1;  // (kept chunks: registers by constant indexes)
+#pragma unroll kUnroll
+  for (int k = 0; k < (KC > 0 ? KC : nch); ++k) {
+    if (KC == 0 || k < nch) {
+      double q[RC];
+      take_q(q);
+      if (k + 1 < nch) {
+        load_f(k + 1);
+        load_q(k + 1);
+      }
+      const double(*s)[RC][64] = s_f[k & 1];
+      if (on) {
 #pragma unroll
-      for (int r = 0; r < RC; ++r) {
-        const int l = k * RC + r + 1;
-        if (l <= n) {
-          const double qr = l < n ? q[r] : qc;  // BC_right_t0 (:845)
-          const double Bn = s[0][r][l64] * ql + s[1][r][l64] * qc + s[2][r][l64] * qr;
-          if (l > 1) {
-            sb[row(l - 1)] = Bc;
-            Bc = Bn - s[3][r][l64] * Bc;
-          } else {
-            Bc = Bn;
+        for (int r = 0; r < RC; ++r) {
+          const int l = k * RC + r + 1;
+          if (l <= n) {
+            const double qr = l < n ? q[r] : qc;  // BC_right_t0 (:845)
+            const double Bn = s[0][r][l64] * ql + s[1][r][l64] * qc + s[2][r][l64] * qr;
+            if (l > 1) {
+              if constexpr (KC > 0) Y[k * RC + r - 1] = Bc;
+              else sb[row(l - 1)] = Bc;
+              Bc = Bn - s[3][r][l64] * Bc;
+            } else {
+              Bc = Bn;
+            }
+            ql = qc;
+            qc = qr;
           }
-          ql = qc;
-          qc = qr;
         }
       }
+      if (k + 1 < nch) put_f(k + 1);
+      wg_lds_barrier();
     }
-    if (k + 1 < nch) put_f(k + 1);
-    wg_lds_barrier();
   }
 
-  // ---- back substitution: chunk k holds rows n - k*RC .. n - k*RC - RC + 1
-  // (row n's right-hand side is Bc)
-  double fb[RPW][2], yn[RC];
+  // ---- back substitution: chunk k holds rows top - k*RC .. top - k*RC - RC + 1
+  // (row n's right-hand side is Bc; kept ones go by the elimination's chunks)
+  const int top = KC > 0 ? nch * RC : n;
+  double fb[RPW][2], yn[KC > 0 ? 1 : RC];
   auto load_b = [&](int k) {
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-      const long long o = row(max(n - k * RC - (w * RPW + r), 1));
+      const int i = max(top - k * RC - (w * RPW + r), 1);
+      const long long o = row(KC > 0 ? min(i, n) : i);
       fb[r][0] = fD[o];
       fb[r][1] = fDU[o];
     }
@@ -186,55 +201,65 @@ __global__ __launch_bounds__(64 * NW) void k_cn_exact(ExactArgs E) {
     }
   };
   auto load_y = [&](int k) {
+    if constexpr (KC == 0) {
 #pragma unroll
-    for (int r = 0; r < RC; ++r) yn[r] = sb[row(min(max(n - k * RC - r, 1), max(n - 1, 1)))];
+      for (int r = 0; r < RC; ++r) yn[r] = sb[row(min(max(n - k * RC - r, 1), max(n - 1, 1)))];
+    }
   };
   double x1 = 0.0, x2 = 0.0;
   load_b(0);
   load_y(0);
   put_b(0);
   wg_lds_barrier();
-  for (int k = 0; k < nch; ++k) {
-    double y[RC], x[RC];
-#pragma unroll
-    for (int r = 0; r < RC; ++r) y[r] = yn[r];
-    if (k + 1 < nch) {
-      load_b(k + 1);
-      load_y(k + 1);
-    }
-    const double(*s)[RC][64] = s_f[k & 1];
-    if (on) {
+#pragma unroll kUnroll
+  for (int j = 0; j < (KC > 0 ? KC : nch); ++j) {
+    const int kk = KC - 1 - j;  // the kept chunk
+    const int k = KC > 0 ? nch - 1 - kk : j;
+    if (KC == 0 || kk < nch) {
+      double y[RC], x[RC];
 #pragma unroll
       for (int r = 0; r < RC; ++r) {
-        const int i = n - k * RC - r;
-        x[r] = 0.0;
-        if (i >= 1) {
-          const double D = s[0][r][l64], DU = s[1][r][l64];
-          double xi;
-          if (i == n) xi = Bc / D;
-          else if (i == n - 1) xi = (y[r] - DU * x1) / D;
-          else xi = (y[r] - DU * x1 - 0.0 * x2) / D;  // (the second super-diagonal is zero)
-          x2 = x1;
-          x1 = xi;
-          x[r] = line_on ? xi : 0.0;
-          if constexpr (!XR) c[ob + os * (long long)(rmin + i)] = x[r];
-        }
+        if constexpr (KC > 0) y[r] = Y[kk * RC + RC - 1 - r];
+        else y[r] = yn[r];
       }
-      if constexpr (XR) {
-        wave_lds();
-#pragma unroll
-        for (int r = 0; r < RC; ++r) tile[l64 * (RC + 1) + (RC - 1 - r)] = x[r];
-        wave_lds();
-        const int lo = n - k * RC - RC;  // row of column 0, less one
+      if (k + 1 < nch) {
+        load_b(k + 1);
+        load_y(k + 1);
+      }
+      const double(*s)[RC][64] = s_f[k & 1];
+      if (on) {
 #pragma unroll
         for (int r = 0; r < RC; ++r) {
-          const int f = r * 64 + l64, ln = f / RC, col = f % RC, i = lo + 1 + col;
-          if (tg.tile * 64 + ln < lines && i >= 1) c[s_row[ln] + rmin + i] = tile[ln * (RC + 1) + col];
+          const int i = top - k * RC - r;
+          x[r] = 0.0;
+          if (i >= 1 && (KC == 0 || i <= n)) {
+            const double D = s[0][r][l64], DU = s[1][r][l64];
+            double xi;
+            if (i == n) xi = Bc / D;
+            else if (i == n - 1) xi = (y[r] - DU * x1) / D;
+            else xi = (y[r] - DU * x1 - 0.0 * x2) / D;  // (the second super-diagonal is zero)
+            x2 = x1;
+            x1 = xi;
+            x[r] = line_on ? xi : 0.0;
+            if constexpr (!XR) c[ob + os * (long long)(rmin + i)] = x[r];
+          }
+        }
+        if constexpr (XR) {
+          wave_lds();
+#pragma unroll
+          for (int r = 0; r < RC; ++r) tile[l64 * (RC + 1) + (RC - 1 - r)] = x[r];
+          wave_lds();
+          const int lo = n - k * RC - RC;  // row of column 0, less one
+#pragma unroll
+          for (int r = 0; r < RC; ++r) {
+            const int f = r * 64 + l64, ln = f / RC, col = f % RC, i = lo + 1 + col;
+            if (tg.tile * 64 + ln < lines && i >= 1) c[s_row[ln] + rmin + i] = tile[ln * (RC + 1) + col];
+          }
         }
       }
+      if (k + 1 < nch) put_b(k + 1);
+      wg_lds_barrier();
     }
-    if (k + 1 < nch) put_b(k + 1);
-    wg_lds_barrier();
   }
   // cells the reference leaves at zero: bins that are not aloft, and cells
   // outside [rmin, rmax] (off lines above)
@@ -243,12 +268,12 @@ __global__ __launch_bounds__(64 * NW) void k_cn_exact(ExactArgs E) {
     if (!on || r < rmin || r > g.rmax) c[ob + os * (long long)(r + 1)] = 0.0;
 }
 
-template <bool XR, int NW, int RC>
+template <bool XR, int NW, int RC, int KC = 0>
 hipError_t launch(hipStream_t s, const ExactArgs &e) {
   const long long lines = (long long)e.A.g.Na * e.A.g.Nb;
   const long long blocks = padded_tiles((lines + 63) / 64) * ((e.A.d.ns + NW - 1) / NW);
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_cn_exact<XR, NW, RC>), dim3((unsigned)blocks), dim3(64, NW), 0, s, e);
+  hipLaunchKernelGGL((k_cn_exact<XR, NW, RC, KC>), dim3((unsigned)blocks), dim3(64, NW), 0, s, e);
   return hipGetLastError();
 }
 
@@ -264,6 +289,19 @@ hipError_t launch_cn_exact(hipStream_t s, const DiffArgs &a, const Dims *orig, d
   if (orig) {
     if (a.d.ns >= 4) return launch<true, 4, 8>(s, e);
     return a.d.ns >= 2 ? launch<true, 2, 8>(s, e) : launch<true, 1, 8>(s, e);
+  }
+  // Right-hand sides kept in registers: z 118 -> 78 us at 240x160x50x8, 504 ->
+  // 315 at 360x240x50x15, 142 -> 97 at 300x120x64x8; 10 chunks (two waves per
+  // SIMD) 3.07 -> 1.92 ms at 1440x720x80x4, 35 us either way for the 80-cell y
+  // lines of 120x80x40x10
+  const int n = a.g.rmax - a.g.rmin + 1;
+  if (n <= 64) {
+    if (a.d.ns >= 4) return launch<false, 4, 8, 8>(s, e);
+    return a.d.ns >= 2 ? launch<false, 2, 8, 8>(s, e) : launch<false, 1, 8, 8>(s, e);
+  }
+  if (n <= 80) {
+    if (a.d.ns >= 4) return launch<false, 4, 8, 10>(s, e);
+    return a.d.ns >= 2 ? launch<false, 2, 8, 10>(s, e) : launch<false, 1, 8, 10>(s, e);
   }
   if (a.d.ns >= 4) return launch<false, 4, 8>(s, e);
   return a.d.ns >= 2 ? launch<false, 2, 8>(s, e) : launch<false, 1, 8>(s, e);
