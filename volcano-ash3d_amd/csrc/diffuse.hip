@@ -88,7 +88,9 @@ __global__ __launch_bounds__(64 * W) void k_line_rows(DiffArgs A, double *lr, Li
         // L, R >= 0 and finite, theta >= 0: every row has D >= 1 + |DL| + |DU|
         // in exact arithmetic (false for NaN too)
         dom = dom && L >= 0.0 && R >= 0.0 && L <= DBL_MAX && R <= DBL_MAX && th >= 0.0;
-        rho = fmax(rho, (fabs(DL) + fabs(DU)) / fabs(D));
+        // (a zero pivot without off-diagonal entries, 0/0, counts as unsafe)
+        const double ratio = (fabs(DL) + fabs(DU)) / fabs(D);
+        rho = fmax(rho, ratio <= DBL_MAX ? ratio : INFINITY);
       }
       kap_c = kap_r;
       k_c = k_r;
