@@ -207,8 +207,12 @@ hipError_t download_levels(hipStream_t s, const Dims &d, bool zero, const double
   }
   while (e == hipSuccess && waited < issued) wait_one();
   if (e != hipSuccess) {
-    std::lock_guard<std::mutex> lk(w.m);
-    w.stop = true;
+    {
+      std::lock_guard<std::mutex> lk(w.m);
+      w.stop = true;
+    }
+    // (no copy may write the caller's array after the call)
+    (void)hipStreamSynchronize(s);
   }
   w.cv.notify_all();
   return e;
