@@ -174,15 +174,10 @@ struct ash3d_tr_ctx {
   bool graph_lu_on[2][3] = {}, graph_lu_full[2][3] = {};
   // sweeps captured without the dgtsv-order alternative, every line being
   // dominant (cap_dom: in the capture under way), and the row factors
-  // (ln_stamp) for which that was seen; the step's own arguments, for an
-  // eager step in place of a replay when it no longer holds
+  // (ln_stamp) for which that was seen; graph_any is the same step with the
+  // alternatives, for replays whose lines are not known to be dominant
   bool cap_dom[3] = {}, graph_dom[2][3] = {};
   long long ln_stamp[3] = {0, 0, 0}, graph_stamp[2][3] = {};
-  struct StepArgs {
-    double dt, imp_fac;
-    int32_t use_diffusion, use_cn;
-    std::vector<int32_t> aloft;
-  } graph_step[2];
   bool graph_tgeom[2] = {false, false};  // the graph reads the transposed geometry
   long long fac_groups = 0;
   // pinned host ring for the source columns: the caller's buffer is copied
@@ -212,7 +207,7 @@ struct ash3d_tr_ctx {
   int met_next = 1, met_count = 0;
   double *dtp = nullptr;                 // Adjust_DT partials, then dz
   // captured glue + step, one graph per step parity
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t graph[2] = {nullptr, nullptr}, graph_any[2] = {nullptr, nullptr};
   unsigned long long *prof = nullptr;    // get_minmax_index slab maxima
   int ts1_state = TS1_EXPLICIT;
   int nb_adv[3] = {4, 4, 4}, nb_diff[3] = {4, 4, 4};  // bins per thread, by direction
@@ -1106,7 +1101,8 @@ int ash3d_tr_destroy(ash3d_tr_ctx *x) {
       if (x->met[a][b]) hipFree(x->met[a][b]);
   if (x->dtp) hipFree(x->dtp);
   for (int k = 0; k < 2; ++k)
-    if (x->graph[k]) hipGraphExecDestroy(x->graph[k]);
+    for (hipGraphExec_t g : {x->graph[k], x->graph_any[k]})
+      if (g) hipGraphExecDestroy(g);
   if (x->prof) hipFree(x->prof);
   for (int k = 0; k < ash3d_tr_ctx::kFluxRing; ++k) {
     if (x->flux_pinned[k]) hipHostFree(x->flux_pinned[k]);
@@ -2018,6 +2014,27 @@ int ash3d_tr_adj_column_load(ash3d_tr_ctx *x, const double *dz, const double *w)
   return 0;
 }
 
+// Captures step_glue + step as a graph.
+static int capture_step(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t use_diffusion, int32_t use_cn,
+                        double imp_fac, const int32_t *is_aloft, hipGraphExec_t *out) {
+  HIPCHK(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
+  x->capturing = true;
+  int rc = ash3d_tr_step_glue(x);
+  if (!rc) rc = ash3d_tr_step(x, itime, dt, use_diffusion, use_cn, imp_fac, is_aloft);
+  x->capturing = false;
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(x->stream, &g);
+  if (rc) {
+    if (g) hipGraphDestroy(g);
+    return rc;
+  }
+  if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "stream capture: %s", hipGetErrorString(e));
+  e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
+  hipGraphDestroy(g);
+  if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "graph instantiation: %s", hipGetErrorString(e));
+  return 0;
+}
+
 int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t use_diffusion, int32_t use_cn,
                            double imp_fac, const int32_t *is_aloft) {
   int rc = check_ctx(x);
@@ -2031,10 +2048,11 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     return fail(ASH3D_TR_EINVAL, "capture after an eager step (transposed geometry not built)");
   HIPCHK(hipStreamSynchronize(x->stream));
   const int slot = itime % 2;
-  if (x->graph[slot]) {
-    HIPCHK(hipGraphExecDestroy(x->graph[slot]));
-    x->graph[slot] = nullptr;
-  }
+  for (hipGraphExec_t *g : {&x->graph[slot], &x->graph_any[slot]})
+    if (*g) {
+      HIPCHK(hipGraphExecDestroy(*g));
+      *g = nullptr;
+    }
   for (int k = 0; k < 3; ++k) x->cap_dom[k] = false;
   x->graph_dtv[slot] = -1.0;
   if (use_diffusion && x->adv_fused && (rc = ensure_dtv(x, dt))) return rc;  // (outside the capture)
@@ -2057,21 +2075,14 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     for (int dir = 0; dir < 3; ++dir) x->cap_dom[dir] = x->cap_dom[dir] && x->cnt_h[dir].ndom == 0;
   }
   for (int k = 0; k < 3; ++k) x->lu_args_set[k] = false;
-  HIPCHK(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-  x->capturing = true;
-  int rc2 = ash3d_tr_step_glue(x);
-  if (!rc2) rc2 = ash3d_tr_step(x, itime, dt, use_diffusion, use_cn, imp_fac, is_aloft);
-  x->capturing = false;
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(x->stream, &g);
-  if (rc2) {
-    if (g) hipGraphDestroy(g);
-    return rc2;
+  if (x->cap_dom[0] || x->cap_dom[1] || x->cap_dom[2]) {
+    bool dom[3];
+    std::copy(x->cap_dom, x->cap_dom + 3, dom);
+    std::fill(x->cap_dom, x->cap_dom + 3, false);
+    if ((rc = capture_step(x, itime, dt, use_diffusion, use_cn, imp_fac, is_aloft, &x->graph_any[slot]))) return rc;
+    std::copy(dom, dom + 3, x->cap_dom);
   }
-  if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "stream capture: %s", hipGetErrorString(e));
-  e = hipGraphInstantiate(&x->graph[slot], g, nullptr, nullptr, 0);
-  hipGraphDestroy(g);
-  if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "graph instantiation: %s", hipGetErrorString(e));
+  if ((rc = capture_step(x, itime, dt, use_diffusion, use_cn, imp_fac, is_aloft, &x->graph[slot]))) return rc;
   for (int k = 0; k < 3; ++k) {
     x->graph_lu_on[slot][k] = x->lu_args_set[k];
     x->graph_lu[slot][k] = x->lu_args[k];
@@ -2080,8 +2091,6 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
     x->graph_stamp[slot][k] = x->ln_stamp[k];
   }
   x->graph_tgeom[slot] = use_diffusion && use_cn;
-  x->graph_step[slot] = {dt, imp_fac, use_diffusion, use_cn,
-                         is_aloft ? std::vector<int32_t>(is_aloft, is_aloft + x->d.ns) : std::vector<int32_t>()};
   return 0;
 }
 
@@ -2102,20 +2111,15 @@ int ash3d_tr_graph_launch(ash3d_tr_ctx *x, int32_t itime) {
     if ((rc = ensure_lr(x, k, a)) || (rc = ensure_lu(x, k, a, x->graph_lu_full[slot][k]))) return rc;
   }
   if ((rc = set_bc1(x, true, nullptr, false))) return rc;
-  // new factors since the lines were seen to be dominant: wait for their
-  // counts; a step with other lines is launched as it is
+  // new factors since the lines were seen to be dominant: unless their
+  // counts have come back and show the same, the device chooses
+  bool dominant = true;
   for (int k = 0; k < 3; ++k) {
     if (!x->graph_dom[slot][k] || x->graph_stamp[slot][k] == x->ln_stamp[k]) continue;
-    HIPCHK(hipStreamSynchronize(x->stream));
-    if (x->cnt_h[k].ndom != 0) {
-      const auto &st = x->graph_step[slot];
-      if ((rc = ash3d_tr_step_glue(x))) return rc;
-      return ash3d_tr_step(x, itime, st.dt, st.use_diffusion, st.use_cn, st.imp_fac,
-                           st.aloft.empty() ? nullptr : st.aloft.data());
-    }
-    x->graph_stamp[slot][k] = x->ln_stamp[k];
+    if (host_ndom(x, k) == 0) x->graph_stamp[slot][k] = x->ln_stamp[k];
+    else dominant = false;
   }
-  HIPCHK(hipGraphLaunch(x->graph[slot], x->stream));
+  HIPCHK(hipGraphLaunch(dominant ? x->graph[slot] : x->graph_any[slot], x->stream));
   x->ts1_state = TS1_MIRROR;
   return 0;
 }
