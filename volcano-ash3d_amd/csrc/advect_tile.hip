@@ -72,6 +72,29 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   const int lim = A.limiter;
   const double dt = A.dt;
   const bool first = r0 == 1, last = r0 + M > N;  // the tile holds cell 1, cell N
+  // A tile with no line or no cell of the box, and a bin that is not aloft,
+  // are stored as zeros and not read (uniform; the outflow of an end of the
+  // line belongs to a tile with cells of the box).  The 3x3x3 box of a
+  // 360x240x50x15 step without diffusion: 641 us, 1057 us with every tile
+  // read.  Bit n - nlo of run: bin n is swept here
+  const uint64_t mask = A.aloft.w[nlo >> 5] | (uint64_t)A.aloft.w[min((nlo >> 5) + 1, kMaxBins / 32 - 1)] << 32;
+  const unsigned group = (1u << (nhi - nlo)) - 1, on = (unsigned)(mask >> (nlo & 31)) & group;
+  const bool in_box = a0 <= g.a1 && a0 + 63 >= g.a0 && b >= g.b0 && b <= g.b1 && r0 <= rmax && r0 + M > rmin;
+  const unsigned run = in_box ? on : 0u;
+  for (unsigned z = group & ~run; z; z &= z - 1) {
+    const int u = __builtin_ctz(z);
+    if (INPL && (on >> u & 1)) __syncthreads();  // (other waves read this tile's edge cells)
+    double *cn = co + d.ncell * (long long)(nlo + u);
+#pragma unroll
+    for (int i = 0; i < M; ++i) (r0 + i <= N ? cn + row(r0 + i) + al : junk)[0] = 0.0;
+  }
+  if (!run) {
+    if (DIR == 2 && first && !repeat)
+      for (int n = nlo; n < nhi; ++n)
+        A.dep[(long long)(a - 1) + (long long)d.nx * ((long long)(b - 1) + (long long)d.ny * n)] =
+            A.of1[(long long)(a + 1) + (long long)(g.Na + 4) * ((long long)(b + 1) + (long long)(g.Nb + 4) * n)];
+    return;
+  }
   // ---- bin-independent terms.  Interface i of the tile is I = r0 + i
   // (0 <= i <= M), between cells I-1 and I
   double sg[M + 1], dtv[M + 1];
@@ -144,16 +167,17 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
       for (int i = 0; i < M + 2; ++i) vs[i] = (fn + row(min(r0 - 1 + i, N + 2)))[al];
     }
   };
-  fetch(nlo);
-  for (int n = nlo; n < nhi; ++n) {
-    const bool on = A.aloft.on(n);
+  fetch(nlo + __builtin_ctz(run));
+  for (unsigned left = run; left; left &= left - 1) {
+    const int n = nlo + __builtin_ctz(left);
     double q[M + 4], vc[M + 2];
 #pragma unroll
     for (int i = 0; i < M + 4; ++i) q[i] = qs[i];
 #pragma unroll
     for (int i = 0; i < M + 2; ++i) vc[i] = DIR == 2 ? wv[i] + vs[i] : 0.0;  // (:171-176)
     const double vf0 = DIR == 2 ? vs[0] : 0.0;
-    fetch(min(n + 1, nhi - 1));
+    const unsigned next = left & (left - 1);
+    fetch(nlo + __builtin_ctz(next ? next : left));
     if (first) q[0] = q[1] = 0.0;
     if (r0 + M + 1 > N) {
 #pragma unroll
@@ -187,10 +211,9 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
       const double upd = -dtv[i] * (fsl + fsr + fss[i + 1] - fss[i]);
       res[i] = q[i + 2] + upd;
     }
-    if (!(plain && on)) {
+    if (!plain) {
 #pragma unroll
-      for (int i = 0; i < M; ++i)
-        res[i] = (on && line_on && r0 + i >= rmin && r0 + i <= rmax) ? res[i] : 0.0;
+      for (int i = 0; i < M; ++i) res[i] = (line_on && r0 + i >= rmin && r0 + i <= rmax) ? res[i] : 0.0;
     }
     if constexpr (INPL) __syncthreads();  // every load of the bin before its first store
     double *cn = co + d.ncell * (long long)n;
@@ -225,13 +248,13 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   const long long ofb = (long long)(g.Na + 4) * (g.Nb + 4);
   if (repeat) return;  // (the last line's increments once)
   for (int n = nlo; n < nhi; ++n) {
-    const bool on = line_on && A.aloft.on(n);
+    const bool swept = line_on && (run >> (n - nlo) & 1);
     const long long of = of0 + ofb * (long long)n;
-    if (at_hi && on) A.of2[of] = A.of2[of] + s_of[(T.bins + n - nlo) * 64 + lane];
+    if (at_hi && swept) A.of2[of] = A.of2[of] + s_of[(T.bins + n - nlo) * 64 + lane];
     if (!first) continue;
-    if (DIR == 2 || (at_lo && on)) {
+    if (DIR == 2 || (at_lo && swept)) {
       double v = A.of1[of];
-      if (at_lo && on) {
+      if (at_lo && swept) {
         v = v + s_of[(n - nlo) * 64 + lane];
         A.of1[of] = v;
       }
