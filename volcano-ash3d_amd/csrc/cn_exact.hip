@@ -85,6 +85,26 @@ __global__ __launch_bounds__(64 * NW, (KC == 8 && NW == 4) ? 3 : 1) void k_cn_ex
   }
   const double th = A.theta, omt = 1.0 - th;
   if (XR) wg_lds_barrier();
+  // cells 1..N of the lines and one bin (its state z) to zero, split over
+  // parts waves (x lines: along the lines)
+  auto clear = [&](double *z, int part, int parts) {
+    if constexpr (XR) {
+      for (int ln = part; ln < 64 && tg.tile * 64 + ln < lines; ln += parts)
+        for (int r = l64; r < N; r += 64) z[s_row[ln] + 2 + r] = 0.0;
+    } else {
+      if (repeat) return;
+      for (int r = 1 + part; r <= N; r += parts) z[ob + os * (long long)(r + 1)] = 0.0;
+    }
+  };
+  // lines outside the box, or bins that are not aloft, throughout the
+  // workgroup (every wave has the same lines; uniform): nothing is read
+  const int b0 = tg.group * NW, b1 = min(b0 + NW, d.ns);
+  bool any_bin = false;
+  for (int q = b0; q < b1; ++q) any_bin = any_bin || A.aloft.on(q);
+  if (!any_bin || __ballot(line_on) == 0) {
+    for (int q = b0; q < b1; ++q) clear((XR ? E.c : A.c0) + (XR ? E.o.ncell : d.ncell) * (long long)q, w, NW);
+    return;
+  }
 
   // ---- elimination: chunk k holds rows k*RC+1 .. k*RC+RC, with the q of
   // each row's right neighbour (cell rmin+l)
@@ -263,9 +283,11 @@ __global__ __launch_bounds__(64 * NW, (KC == 8 && NW == 4) ? 3 : 1) void k_cn_ex
   }
   // cells the reference leaves at zero: bins that are not aloft, and cells
   // outside [rmin, rmax] (off lines above)
-  if (!exists || repeat) return;
+  if (!exists) return;
+  if (!on) return clear(c, 0, 1);
+  if (repeat) return;
   for (int r = 1; r <= N; ++r)
-    if (!on || r < rmin || r > g.rmax) c[ob + os * (long long)(r + 1)] = 0.0;
+    if (r < rmin || r > g.rmax) c[ob + os * (long long)(r + 1)] = 0.0;
 }
 
 template <bool XR, int NW, int RC, int KC = 0>
