@@ -77,8 +77,7 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   // line belongs to a tile with cells of the box).  The 3x3x3 box of a
   // 360x240x50x15 step without diffusion: 641 us, 1057 us with every tile
   // read.  Bit n - nlo of run: bin n is swept here
-  const uint64_t mask = A.aloft.w[nlo >> 5] | (uint64_t)A.aloft.w[min((nlo >> 5) + 1, kMaxBins / 32 - 1)] << 32;
-  const unsigned group = (1u << (nhi - nlo)) - 1, on = (unsigned)(mask >> (nlo & 31)) & group;
+  const unsigned group = (1u << (nhi - nlo)) - 1, on = A.aloft.bits(nlo, nhi);
   const bool in_box = a0 <= g.a1 && a0 + 63 >= g.a0 && b >= g.b0 && b <= g.b1 && r0 <= rmax && r0 + M > rmin;
   const unsigned run = in_box ? on : 0u;
   for (unsigned z = group & ~run; z; z &= z - 1) {

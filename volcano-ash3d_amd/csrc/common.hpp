@@ -38,6 +38,12 @@ constexpr int kMaxBins = 1024;
 struct AloftMask {
   uint32_t w[kMaxBins / 32];
   __host__ __device__ inline bool on(int n) const { return (w[n >> 5] >> (n & 31)) & 1u; }
+  // bins lo .. hi-1 (at most 32) as bits 0, 1, ...: two words read, however many bins
+  __device__ inline uint32_t bits(int lo, int hi) const {
+    const int q = lo >> 5;
+    const uint64_t m = w[q] | (uint64_t)w[q + 1 < kMaxBins / 32 ? q + 1 : q] << 32;
+    return (uint32_t)(m >> (lo & 31)) & (uint32_t)((1ull << (hi - lo)) - 1);
+  }
 };
 
 // Geometry of one sweep direction: lines of length N along dir, transverse
