@@ -218,8 +218,10 @@ enum {
   ASH3D_TUNE_PART_SHAPE_X = 9, /* tile shape of the partitioned solves (0 or 1; defaults 1, 1, 0), x lines */
   ASH3D_TUNE_PART_SHAPE_Y = 10,
   ASH3D_TUNE_PART_SHAPE_Z = 11,
-  /* streamed y/z advection (in-place sweeps along more than 64 cells; the
-   * others run in register tiles, which take no setting): 0 cuts the lines of a workgroup into segments;
+  /* streamed y/z advection (in-place sweeps along more than 64 cells, some
+   * in-place z sweeps of shorter lines, and boxes that reach the top without
+   * starting at the bottom; the others run in register tiles, which take no
+   * setting): 0 cuts the lines of a workgroup into segments;
    * 1..4 gives each wave of a workgroup one bin group of the same whole
    * lines, so the per-cell fields are read once for all of them */
   ASH3D_TUNE_ADV_GROUPS_Y = 12,

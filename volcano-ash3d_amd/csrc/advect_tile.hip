@@ -65,7 +65,7 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   const bool plain = rmin == 1 && rmax == N && g.a0 == 1 && g.a1 == g.Na && g.b0 == 1 && g.b1 == g.Nb;
   const long long sL = line_stride(d, DIR), base = line_base(d, DIR, a0, b);
   auto row = [&](int r) { return base + sL * (long long)(r + 1); };  // uniform; + al
-  double *junk = A.junk + lane + 64 * w + 512 * (int)(vb % (kJunk / 512));
+  double *junk = A.junk + lane + 64 * (int)(vb % (kJunk / 64));  // (of the wave with the line's last cells)
   const int nlo = tg.group * T.bins, nhi = min(nlo + T.bins, d.ns);
   const double *c = A.c0;
   double *co = A.cout;
@@ -264,12 +264,16 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   }
 }
 
+// most threads of a workgroup (in place: the waves of a line of 60, 48 or 64 cells)
+template <int M, bool INPL>
+constexpr int kTileThreads = !INPL ? 256 : M == 5 ? 768 : 512;
+
 template <int DIR, int M, int LIM, bool TOPO, bool INPL>
-__global__ __launch_bounds__(INPL ? 512 : 256) void k_advect_tile(TileArgs T) {
+__global__ __launch_bounds__((kTileThreads<M, INPL>)) void k_advect_tile(TileArgs T) {
   advect_tile_body<DIR, M, LIM, TOPO, INPL>(T, blockIdx.x, gridDim.x);
 }
 template <int DIR, int M, int LIM, bool TOPO, bool INPL>
-__global__ __launch_bounds__(INPL ? 512 : 256) void k_advect_tile_batch(
+__global__ __launch_bounds__((kTileThreads<M, INPL>)) void k_advect_tile_batch(
     const ASH3D_CONSTANT TileArgs *__restrict__ args, const ASH3D_CONSTANT int *__restrict__ member,
     const ASH3D_CONSTANT long long *__restrict__ first) {
   const int m = member[blockIdx.x];
@@ -309,35 +313,68 @@ hipError_t tile_lim(hipStream_t s, const AdvArgs &a, LaunchSpec *sp) {
 }  // namespace
 
 // The y or z sweep of a in register tiles: issued (or described in sp), or
-// hipErrorInvalidValue where the streamed kernel runs it: in place a line
-// of more than 64 cells (its waves would not fit one workgroup), and the z
-// box that ends at the top without starting at the bottom (its top outflow
-// is the update of cell ncells+1, src/AdvectionVert_DCU.f90:309-311).
+// hipErrorInvalidValue where the streamed kernel runs it (advect_tile_applies).
 //
-// Five cells per wave: 168 VGPRs, three waves per SIMD (with topography 197,
-// two).  Measured on 360x240x50x15 (64.8 M bin-cells, superbee): y 300 us,
-// z 467 us against 331 and 481 streamed; 1440x720x80x4: 1.55 and 2.45 ms
-// (4.7 and 4.3 TB/s of the compulsory bytes) against 2.33 (y streamed) and,
-// for the fused second horizontal + z pass, 4.2 ms; 120x80x40x10: 18 and 24
-// us against 47 and 55.  Three, four or six cells: y 315, 304, 300 us, z 492,
-// 472, 478 us on the first grid.  One, two or three waves per workgroup
-// instead of four, tiles of 64 lines cut across the ends of the rows (no
-// idle lanes, but neighbouring tiles further apart in time: y 335 us),
-// non-temporal stores (y 343 us): no gain.
+// Out of place: five cells per wave, 162 VGPRs, three waves per SIMD (with
+// topography 194, two).  Measured on 360x240x50x15 (64.8 M bin-cells,
+// superbee): y 300 us, z 467 us against 331 and 481 streamed; 1440x720x80x4:
+// 1.55 and 2.45 ms (4.7 and 4.3 TB/s of the compulsory bytes) against 2.33 (y
+// streamed) and, for the fused second horizontal + z pass, 4.2 ms;
+// 120x80x40x10: 18 and 24 us against 47 and 55.  Three, four or six cells: y
+// 315, 304, 300 us, z 492, 472, 478 us on the first grid.  One, two or three
+// waves per workgroup instead of four, tiles of 64 lines cut across the ends
+// of the rows (no idle lanes, but neighbouring tiles further apart in time: y
+// 335 us), non-temporal stores (y 343 us): no gain.
+//
+// In place a line's N / M waves are one workgroup, and as many workgroups as
+// fit a CU overlap one's loads with another's barrier: five cells (12 waves
+// per CU, up to 60 cells) unless eight (8 waves) let two workgroups in where
+// the waves of five cells are as many and shorter (21 to 32 cells: z of
+// 656x58x31x10 90 us against 105 with five and 122 with six), or lines of 41
+// to 48 cells fill 7 or 8 waves of six (z of 565x28x45x20 118 us against 124
+// with five and eight).  z of 46x26x53x2, 76x22x49x9, 240x160x50x9: 17, 21 and
+// 158 us against 58, 58 and 193 streamed.
 hipError_t advect_tile(hipStream_t s, const AdvArgs &a, LaunchSpec *sp) {
   const bool inpl = a.cout == a.c0;
-  if (!advect_tile_applies(a.g, inpl)) return hipErrorInvalidValue;
-  if (a.g.dir == 2) {
-    if (!inpl) return tile_lim<2, 5, false, false>(s, a, sp);
-    return a.g.N <= 48 ? tile_lim<2, 6, false, true>(s, a, sp) : tile_lim<2, 8, false, true>(s, a, sp);
+  const int N = a.g.N;
+  if (!advect_tile_applies(a.g, a.d.ns, inpl)) return hipErrorInvalidValue;
+  if (!inpl) {
+    if (a.g.dir == 2) return tile_lim<2, 5, false, false>(s, a, sp);
+    return a.deld ? tile_lim<1, 5, true, false>(s, a, sp) : tile_lim<1, 5, false, false>(s, a, sp);
   }
-  if (!inpl) return a.deld ? tile_lim<1, 5, true, false>(s, a, sp) : tile_lim<1, 5, false, false>(s, a, sp);
-  return a.deld ? tile_lim<1, 8, true, true>(s, a, sp) : tile_lim<1, 8, false, true>(s, a, sp);
+  const bool six = N > 40 && N <= 48, eight = (N > 20 && N <= 32) || N > 60;
+  if (a.g.dir == 2) {
+    if (six) return tile_lim<2, 6, false, true>(s, a, sp);
+    return eight ? tile_lim<2, 8, false, true>(s, a, sp) : tile_lim<2, 5, false, true>(s, a, sp);
+  }
+  // (with topography five cells take more than three waves' registers)
+  if (a.deld) return N <= 48 ? tile_lim<1, 6, true, true>(s, a, sp) : tile_lim<1, 8, true, true>(s, a, sp);
+  if (six) return tile_lim<1, 6, false, true>(s, a, sp);
+  return eight ? tile_lim<1, 8, false, true>(s, a, sp) : tile_lim<1, 5, false, true>(s, a, sp);
 }
 
-bool advect_tile_applies(const LineGeom &g, bool in_place) {
+// Streamed instead: the z box that ends at the top without starting at the
+// bottom (its top outflow is the update of cell ncells+1, src/
+// AdvectionVert_DCU.f90:309-311); in place lines of more than 64 cells (their
+// waves would not fit one workgroup), and z lines with enough tiles to fill
+// the chip either way, where a tile's set-up serves few bins (one, or two, four
+// or eight, which the streamed kernel takes in whole pairs), or long lines have
+// many bins.  Tile of five, six or eight cells against streamed: 497x387x54x2
+// 271 and 236 us, 354x247x35x2 72 and 63, 334x221x50x4 163 and 149,
+// 663x253x31x1 78 and 68, 607x194x51x1 104 and 82, 134x180x41x8 100 and 85,
+// 240x160x50x8 137 and 131, 360x240x50x15 532 and 504, 426x189x63x15 603 and
+// 563; below the bounds 552x94x60x2 73 and 89, 389x90x58x1 40 and 46,
+// 41x253x45x8 49 and 59, 65x25x58x15 44 and 91.
+bool advect_tile_applies(const LineGeom &g, int ns, bool in_place) {
   if (g.dir == 0 || (g.dir == 2 && g.rmax == g.N && g.rmin != 1)) return false;
-  return !in_place || g.N <= 64;
+  if (!in_place) return true;
+  if (g.N > 64) return false;
+  if (g.dir == 1) return true;
+  const long long tiles = (long long)((g.Na + 63) / 64) * g.Nb;
+  if (ns == 1 && g.N > 20 && tiles >= 768) return false;
+  if ((ns == 2 || ns == 4) && g.N > 32 && tiles >= 1024) return false;
+  if (ns == 8 && g.N > 32 && tiles >= 512) return false;
+  return !(ns > 12 && g.N > 48 && tiles >= 1024);
 }
 
 }  // namespace ash3d

@@ -461,8 +461,8 @@ int sweep_advect(ash3d_tr_ctx *x, int dir, double dt, const int32_t *is_aloft, c
 // here before the x sweep.  Not for a periodic step without diffusion,
 // whose x ghosts in ts0 stay observable.
 bool advect_through_ts1(const ash3d_tr_ctx *x, const int32_t *bounds, bool zg) {
-  return (zg || !x->periodic) && advect_tile_applies(make_line_geom(x->d, 1, bounds), false) &&
-         advect_tile_applies(make_line_geom(x->d, 2, bounds), false);
+  return (zg || !x->periodic) && advect_tile_applies(make_line_geom(x->d, 1, bounds), x->d.ns, false) &&
+         advect_tile_applies(make_line_geom(x->d, 2, bounds), x->d.ns, false);
 }
 AdvArgs through_ts1_args(ash3d_tr_ctx *x, int dir, double dt, const int32_t *is_aloft, const int32_t *bounds,
                          bool x_first) {

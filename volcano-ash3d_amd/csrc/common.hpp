@@ -292,7 +292,7 @@ hipError_t spec_advect_hz(const AdvArgs &h, const AdvArgs &z, LaunchSpec *sp);
 // y and z sweeps in register tiles (advect_tile.hip): issue the launch, or
 // describe it in sp; hipErrorInvalidValue where advect_tile_applies is false
 hipError_t advect_tile(hipStream_t s, const AdvArgs &a, LaunchSpec *sp);
-bool advect_tile_applies(const LineGeom &g, bool in_place);
+bool advect_tile_applies(const LineGeom &g, int ns, bool in_place);
 hipError_t launch_advect_x_rows(hipStream_t s, const AdvArgs &a);
 // the launch launch_advect_x_rows would issue (hipErrorInvalidValue: the
 // row needs the streamed kernel)
