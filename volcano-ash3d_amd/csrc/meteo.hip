@@ -67,6 +67,29 @@ __device__ inline double block_max(double v, double *sh) {
   return r;
 }
 
+// The largest of the bins' |at(n)|, up to eight loads in flight; the last
+// group is the smallest power of two that holds the bins left (its loads past
+// the last bin repeat that one's): adjust_dt at 720x360x70x1 392 us, 426 with
+// eight loads throughout.
+template <int U, typename T, typename F>
+__device__ __forceinline__ T raise_by_bins(T m, int n0, int ns, F &&at) {
+  T v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = at(min(n0 + u, ns - 1));
+#pragma unroll
+  for (int u = 0; u < U; ++u) m = fmax(m, fabs(v[u]));
+  return m;
+}
+template <typename T, typename F>
+__device__ __forceinline__ T max_over_bins(int ns, F &&at) {
+  T m = 0;
+  int n = 0;
+  for (; ns - n > 4; n += 8) m = raise_by_bins<8>(m, n, ns, at);
+  if (ns - n > 2) return raise_by_bins<4>(m, n, ns, at);
+  if (ns - n == 2) return raise_by_bins<2>(m, n, ns, at);
+  return ns > n ? raise_by_bins<1>(m, n, ns, at) : m;
+}
+
 // Per-block partials of Adjust_DT over the interior cells:
 // [0] vxmax_dx (lon-lat) or max|vx| (projected), [1] the same for y,
 // [2] vzmax_dz, [3] min of the diffusion times (negated, so that all four
@@ -79,19 +102,31 @@ struct DtArgs {
   double *partial;  // [blocks][4]
 };
 
+template <bool PACKED>
 __global__ __launch_bounds__(kRed) void k_dt_partials(DtArgs A) {
   __shared__ double sh[kRed];
   const Dims d = A.d;
   const long long n3 = (long long)d.nx * d.ny * d.nz;
   const long long kxs = d.nx + 2, kxys = (long long)(d.nx + 2) * (d.ny + 2);
   double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = -INFINITY;
-  // a wave takes 64 cells of an x row at a time
-  const unsigned chunks = (unsigned)(d.nx + 63) / 64, items = chunks * (unsigned)d.ny * (unsigned)d.nz;
-  for (unsigned it = blockIdx.x * (kRed / 64) + threadIdx.x / 64; it < items; it += gridDim.x * (kRed / 64)) {
-    const int i = (int)(it % chunks) * 64 + (int)(threadIdx.x & 63) + 1;
-    const unsigned row = it / chunks;
-    const int j = (int)(row % (unsigned)d.ny) + 1, k = (int)(row / (unsigned)d.ny) + 1;
-    if (i > d.nx) continue;
+  // a wave takes 64 cells of an x row at a time (PACKED: 64 cells in the order
+  // of the unpadded arrays, over the ends of the rows)
+  const unsigned nx = (unsigned)d.nx, ny = (unsigned)d.ny, chunks = (nx + 63) / 64;
+  const long long items = PACKED ? (n3 + 63) / 64 : (long long)chunks * ny * d.nz;
+  for (long long it = (long long)blockIdx.x * (kRed / 64) + threadIdx.x / 64; it < items; it += gridDim.x * (kRed / 64)) {
+    const unsigned lane = threadIdx.x & 63;
+    unsigned row, qi;
+    if constexpr (PACKED) {
+      const long long c = 64 * it + lane;
+      row = n3 <= 0xffffffffLL - 64 ? (unsigned)c / nx : (unsigned)(c / nx);
+      qi = (unsigned)(c - (long long)row * nx);
+      if (row >= ny * (unsigned)d.nz) continue;
+    } else {
+      row = (unsigned)it / chunks;
+      qi = ((unsigned)it - row * chunks) * 64 + lane;
+      if (qi >= nx) continue;
+    }
+    const int i = (int)qi + 1, j = (int)(row % ny) + 1, k = (int)(row / ny) + 1;
     const long long m = (long long)d.nx * row + (i - 1);
     const long long o = d.p3(i, j, k);
     const double kap = A.kap[o];
@@ -105,14 +140,7 @@ __global__ __launch_bounds__(kRed) void k_dt_partials(DtArgs A) {
         r0 = fmax(r0, (double)fabsf(A.mx[m]));
         r1 = fmax(r1, (double)fabsf(A.my[m]));
       }
-      float vfm = 0.0f;
-      for (int n0 = 0; n0 < d.ns; n0 += 8) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = A.mf[m + n3 * min(n0 + u, d.ns - 1)];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) vfm = fmaxf(vfm, fabsf(v[u]));
-      }
+      const float vfm = max_over_bins<float>(d.ns, [&](int n) { return A.mf[m + n3 * n]; });
       r2 = fmax(r2, (double)(fabsf(A.mz[m]) + vfm) * MPS_2_KMPHR / A.dz[k - 1]);
     } else {
       if (A.latlon) {
@@ -124,14 +152,7 @@ __global__ __launch_bounds__(kRed) void k_dt_partials(DtArgs A) {
         r0 = fmax(r0, fabs(A.vx[o]));
         r1 = fmax(r1, fabs(A.vy[o]));
       }
-      double vfm = 0.0;
-      for (int n0 = 0; n0 < d.ns; n0 += 8) {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = A.vf[o + d.ncell * min(n0 + u, d.ns - 1)];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) vfm = fmax(vfm, fabs(v[u]));
-      }
+      const double vfm = max_over_bins<double>(d.ns, [&](int n) { return A.vf[o + d.ncell * n]; });
       r2 = fmax(r2, (fabs(A.vz[o]) + vfm) / A.dz[k - 1]);
     }
     if (A.diffusion) {
@@ -246,7 +267,12 @@ hipError_t launch_dt_partials(hipStream_t s, const Dims &d, int latlon, int met,
                               double *partial) {
   DtArgs A{d, latlon, met, diffusion, vx, vy, vz, vf, kap, sx, sy, sz, kx, ky, kz, dz,
            met_next[0], met_next[1], met_next[2], met_next[3], partial};
-  hipLaunchKernelGGL(k_dt_partials, dim3(dt_partial_blocks(d)), dim3(kRed), 0, s, A);
+  // Rows that leave a fifth of the lanes or more idle are packed: adjust_dt at
+  // 30x1000x20x3 50.6 us, 57.0 by rows, 65x65x33x3 42.5 and 45.5; by rows
+  // 360x240x50x15 195 us, 213 packed (the divisions of every lane)
+  const bool packed = 5 * (long long)d.nx <= 4 * 64 * (((long long)d.nx + 63) / 64);
+  if (packed) hipLaunchKernelGGL((k_dt_partials<true>), dim3(dt_partial_blocks(d)), dim3(kRed), 0, s, A);
+  else hipLaunchKernelGGL((k_dt_partials<false>), dim3(dt_partial_blocks(d)), dim3(kRed), 0, s, A);
   return hipGetLastError();
 }
 
