@@ -16,25 +16,29 @@ namespace {
 constexpr double MPS_2_KMPHR = 3.6;  // src/Ash3d_VariableModules.f90:286
 
 // v_pd(1:nx,1:ny,1:nz) = (real(last) + real(next - last) * frac) * 3.6,
-// the difference in FP32 as the _sp arrays give it.  A wave per x row of
-// the unpadded FP32 arrays: blockIdx.y 0 the rows of the three winds, n the
-// rows of bin n - 1's fall speed.  Bound by HBM bandwidth: the fall speeds
-// of 360x240x50x15 (1.04 GB) in 215 us against 260 us with the indices of
-// every cell divided out.
-constexpr int kRow = 256;  // threads per workgroup: 4 rows
+// the difference in FP32 as the _sp arrays give it.  A wave takes SEG cells of
+// an x row of the unpadded FP32 arrays: blockIdx.y 0 the three winds, n bin
+// n - 1's fall speed.  Bound by HBM bandwidth.  With fall speeds 256 cells,
+// four loads of a bin in flight: 1.0 GB of 360x240x50x15 in 238 us, 250 with
+// a whole row per wave and 298 with the indices of every cell divided out.
+// The winds alone 64 cells: 720x360x70 173 us, 201 with a whole row.
+constexpr int kRow = 256;  // threads per workgroup
 
+template <int SEG>
 __global__ __launch_bounds__(kRow) void k_met_interp(Dims d, const float *__restrict__ lx, const float *__restrict__ ly,
                                                     const float *__restrict__ lz, const float *__restrict__ lf,
                                                     const float *__restrict__ nx_, const float *__restrict__ ny_,
                                                     const float *__restrict__ nz_, const float *__restrict__ nf,
                                                     double frac, double *vx, double *vy, double *vz, double *vf) {
-  const unsigned r = blockIdx.x * (kRow / 64) + threadIdx.x / 64;
+  const unsigned segs = (unsigned)(d.nx + SEG - 1) / SEG;
+  const unsigned item = blockIdx.x * (kRow / 64) + threadIdx.x / 64, r = segs == 1 ? item : item / segs;
   if (r >= (unsigned)d.ny * (unsigned)d.nz) return;
-  const int lane = threadIdx.x & 63;
+  const int i0 = (int)(item - r * segs) * SEG + (int)(threadIdx.x & 63), end = min(i0 + SEG, d.nx);
   const long long o = d.p3(1, (int)(r % (unsigned)d.ny) + 1, (int)(r / (unsigned)d.ny) + 1);
   const long long m = (long long)d.nx * r;
   if (blockIdx.y == 0) {
-    for (int i = lane; i < d.nx; i += 64) {
+#pragma unroll 2
+    for (int i = i0; i < end; i += 64) {
       const float ax = lx[m + i], ay = ly[m + i], az = lz[m + i];
       const float dx = nx_[m + i] - ax, dy = ny_[m + i] - ay, dz = nz_[m + i] - az;
       vx[o + i] = ((double)ax + (double)dx * frac) * MPS_2_KMPHR;
@@ -46,7 +50,7 @@ __global__ __launch_bounds__(kRow) void k_met_interp(Dims d, const float *__rest
     const long long mf = m + (long long)d.nx * d.ny * d.nz * n;
     double *w = vf + o + d.ncell * (long long)n;
 #pragma unroll 4
-    for (int i = lane; i < d.nx; i += 64) {
+    for (int i = i0; i < end; i += 64) {
       const float a = lf[mf + i], dv = nf[mf + i] - a;
       w[i] = ((double)a + (double)dv * frac) * MPS_2_KMPHR;
     }
@@ -247,10 +251,14 @@ __global__ void k_zero_u64(unsigned long long *p, int n) {
 
 hipError_t launch_met_interp(hipStream_t s, const Dims &d, const float *const last[4], const float *const next[4],
                              double frac, bool with_vf, double *vx, double *vy, double *vz, double *vf) {
-  const unsigned rows = (unsigned)d.ny * (unsigned)d.nz;
-  hipLaunchKernelGGL(k_met_interp, dim3((rows + kRow / 64 - 1) / (kRow / 64), with_vf ? 1 + d.ns : 1), dim3(kRow), 0,
-                     s, d, last[0], last[1], last[2], last[3], next[0], next[1], next[2], next[3], frac, vx, vy, vz,
-                     vf);
+  const int seg = with_vf ? 256 : 64;
+  const long long items = (long long)d.ny * d.nz * ((d.nx + seg - 1) / seg);
+  const long long blocks = (items + kRow / 64 - 1) / (kRow / 64);
+  if (blocks > 0x3fffffffLL) return hipErrorInvalidValue;  // (item numbers of 32 bits)
+  const dim3 grid((unsigned)blocks, with_vf ? 1 + d.ns : 1);
+  auto *k = with_vf ? k_met_interp<256> : k_met_interp<64>;
+  hipLaunchKernelGGL(k, grid, dim3(kRow), 0, s, d, last[0], last[1], last[2], last[3], next[0], next[1], next[2],
+                     next[3], frac, vx, vy, vz, vf);
   return hipGetLastError();
 }
 
