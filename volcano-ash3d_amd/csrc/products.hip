@@ -28,43 +28,85 @@ constexpr double M_2_MM = 1.0e3;     // :281
 
 // Columns in workgroups of kCol columns (lanes along x) x kWaves waves: the
 // waves take the levels of a chunk of kChunk between them, each level's sum
-// over the bins in the reference's order with kAhead bins' loads in flight,
+// over the bins in the reference's order with eight bins' loads in flight,
 // into LDS; then the first wave folds the chunk's levels upward.  One pass
 // over the state, bound by HBM bandwidth: 518 MB of a 360x240x50x15 state in
 // 125 us (products) and 120 us (column load), against 349 and 338 us with
 // one thread per column, which kept a load or two in flight per lane.
-constexpr int kCol = 64, kWaves = 8, kChunk = 16, kAhead = 8;
+constexpr int kCol = 64, kWaves = 8, kChunk = 16;
+
+// s + the U bins of p from n0 on, in order, their loads in flight together
+// (those past the last bin repeat that one's and are not added)
+template <int U>
+__device__ __forceinline__ double add_bins(double s, const double *p, const Dims &d, int n0) {
+  double v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = p[d.ncell * (long long)min(n0 + u, d.ns - 1)];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (n0 + u < d.ns) s += v[u];
+  return s;
+}
 
 // The sums over the bins of levels k0 .. k0+kChunk-1 (those <= nz) of the
-// workgroup's columns into sum[level - k0][lane]; o: the column's offset at
-// level 0 (c null: zeros).  Ends with a barrier.
-__device__ inline void level_sums(const Dims &d, const double *c, long long o, int k0, double (*sum)[kCol]) {
+// workgroup's columns into sum[level - k0][lane], and what they add to the load
+// into term (formed here: one wave folds all levels, and its divisions would
+// hold up the others); o: the column's offset at level 0 (c null: zeros; sum
+// null: not stored).  The last group of bins is the smallest power of two
+// that holds the bins left (column load at 100x200x60x2 44 us, 50 with eight
+// loads throughout).  Ends with a barrier.
+__device__ inline void level_sums(const Dims &d, const double *c, long long o, const double *dz, int k0, double (*sum)[kCol],
+                                  double (*term)[kCol]) {
   const int l = threadIdx.x, w = threadIdx.y;
-  for (int q = w; q < kChunk && k0 + q <= d.nz; q += kWaves) {
+#pragma unroll
+  for (int q = w; q < kChunk; q += kWaves) {
+    if (k0 + q > d.nz) break;
     double s = 0.0;
     if (c != nullptr) {
       const double *p = c + o + d.sz * (long long)(k0 + q);
-      for (int n0 = 0; n0 < d.ns; n0 += kAhead) {
-        double v[kAhead];
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) v[u] = p[d.ncell * (long long)min(n0 + u, d.ns - 1)];
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u)
-          if (n0 + u < d.ns) s += v[u];
-      }
+      int n = 0;
+      for (; d.ns - n > 4; n += 8) s = add_bins<8>(s, p, d, n);
+      if (d.ns - n > 2) s = add_bins<4>(s, p, d, n);
+      else if (d.ns - n == 2) s = add_bins<2>(s, p, d, n);
+      else if (d.ns > n) s = add_bins<1>(s, p, d, n);
     }
-    sum[q][l] = s;
+    if (sum) sum[q][l] = s;
+    term[q][l] = s * dz[k0 + q - 1] / 1.0e3;
   }
   __syncthreads();
 }
 
+// The same for one column by its own thread, folded upward eight levels at a
+// time: fold(k, sum over the bins, its term of the load).
+constexpr int kWhole = 256;  // columns (threads) of a workgroup
+template <typename F>
+__device__ __forceinline__ void whole_column(const Dims &d, const double *c, long long o, const double *dz, F &&fold) {
+  for (int k0 = 1; k0 <= d.nz; k0 += 8) {
+    double s[8] = {};
+    if (c != nullptr)
+      for (int n = 0; n < d.ns; ++n) {
+        const double *p = c + o + d.ncell * (long long)n;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[q] += p[d.sz * (long long)min(k0 + q, d.nz)];
+      }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (k0 + q <= d.nz) fold(k0 + q, s[q], s[q] * dz[k0 + q - 1] / 1.0e3);
+  }
+}
+// Few bins of many columns: a workgroup's waves would meet at a barrier for
+// every two loads a lane.  Products and column load of 720x360x70x1 42 and 26
+// us (the waves of a workgroup 82 and 51), 720x360x30x2 32 and 22 (45 and
+// 30), 1440x300x30x4 89 and 77 (111 and 85).
+inline bool whole_columns(const Dims &d) { return d.ns <= 4 && (long long)d.nx * d.ny >= 1 << 17; }
+
 // out: 5 planes of nx*ny doubles (cloud load, max concentration, max
 // height, min height, deposit thickness) then 2 planes of int32 masks.
-__global__ __launch_bounds__(kCol *kWaves) void k_products(ProdArgs P) {
-  __shared__ double sum[2][kChunk][kCol];
+template <bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? kWhole : kCol *kWaves) void k_products(ProdArgs P) {
   const Dims d = P.d;
   const unsigned nxy = (unsigned)d.nx * (unsigned)d.ny;
-  const unsigned t = blockIdx.x * kCol + threadIdx.x, tt = min(t, nxy - 1);
+  const unsigned t = blockIdx.x * (WHOLE ? kWhole : kCol) + threadIdx.x, tt = min(t, nxy - 1);
   const int i = (int)(tt % (unsigned)d.nx) + 1, j = (int)(tt / (unsigned)d.nx) + 1;
   const long long o = d.p3(i, j, 0);
   double *load = P.out, *maxc = P.out + nxy, *maxh = maxc + nxy, *minh = maxh + nxy, *thick = minh + nxy;
@@ -72,19 +114,29 @@ __global__ __launch_bounds__(kCol *kWaves) void k_products(ProdArgs P) {
   // ConcentrationCalculator, columns of the box imin..imax x jmin..jmax
   double L = 0.0, H = 0.0, B = 100.0, C = 0.0, tcmax = 0.0;
   bool first_le = false;
-  for (int k0 = 1, par = 0; k0 <= d.nz; k0 += kChunk, par ^= 1) {
-    level_sums(d, P.c, o, k0, sum[par]);
-    if (threadIdx.y != 0) continue;
-    for (int k = k0; k < k0 + kChunk && k <= d.nz; ++k) {
-      const double tc = sum[par][k - k0][threadIdx.x];  // sum(concen_pd(i,j,k,1:n_gs_max,ts1)), bins in order
-      L = L + tc * P.dz[k - 1] / 1.0e3;
-      if (tc >= P.cloudcon) H = P.zcc[k - 1] + 0.5 * P.dz[k - 1];
-      // the top-down scan keeps the lowest level at or below the threshold
-      if (tc <= P.cloudcon && !first_le) {
-        B = P.zcc[k - 1] - 0.5 * P.dz[k - 1];
-        first_le = true;
-      }
-      tcmax = (k == 1) ? tc : fmax(tcmax, tc);  // maxval(TotalConcentration(:))
+  auto fold = [&](int k, double tc, double term) {  // tc: sum(concen_pd(i,j,k,1:n_gs_max,ts1)), bins in order
+    // (heights of every level, not only of the columns that take them: loads
+    // under a lane's condition would wait one after the other)
+    const double zc = P.zcc[k - 1], hdz = 0.5 * P.dz[k - 1], top = zc + hdz, base = zc - hdz;
+    L = L + term;
+    if (tc >= P.cloudcon) H = top;
+    // the top-down scan keeps the lowest level at or below the threshold
+    if (tc <= P.cloudcon && !first_le) {
+      B = base;
+      first_le = true;
+    }
+    tcmax = (k == 1) ? tc : fmax(tcmax, tc);  // maxval(TotalConcentration(:))
+  };
+  if constexpr (WHOLE) {
+    whole_column(d, P.c, o, P.dz, fold);
+  } else {
+    __shared__ double sum[2][kChunk][kCol], term[2][kChunk][kCol];
+    for (int k0 = 1, par = 0; k0 <= d.nz; k0 += kChunk, par ^= 1) {
+      level_sums(d, P.c, o, P.dz, k0, sum[par], term[par]);
+      if (threadIdx.y != 0) continue;
+#pragma unroll 4
+      for (int k = k0; k < min(k0 + kChunk, d.nz + 1); ++k)
+        fold(k, sum[par][k - k0][threadIdx.x], term[par][k - k0][threadIdx.x]);
     }
   }
   if (t >= nxy) return;
@@ -111,7 +163,8 @@ __global__ __launch_bounds__(kCol *kWaves) void k_products(ProdArgs P) {
     maxh[t] = H;
     minh[t] = B;
     mcloud[t] = mask;
-  } else if (threadIdx.y == 1) {
+  }
+  if (WHOLE || threadIdx.y == 1) {
     // AshThicknessCalculator, every column
     double s = 0.0;  // sum(DepositGranularity(i,j,1:n_gs_max))
     for (int n = 0; n < d.ns; ++n) s += P.dep[t + (long long)nxy * n];
@@ -122,17 +175,22 @@ __global__ __launch_bounds__(kCol *kWaves) void k_products(ProdArgs P) {
 }
 
 // CloudLoad of every column (no threshold): out(nx, ny)
-__global__ __launch_bounds__(kCol *kWaves) void k_column_load(Dims d, const double *c0, const double *dz,
-                                                             double *out) {
-  __shared__ double sum[2][kChunk][kCol];
+template <bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? kWhole : kCol *kWaves) void k_column_load(Dims d, const double *c0,
+                                                                              const double *dz, double *out) {
   const unsigned nxy = (unsigned)d.nx * (unsigned)d.ny;
-  const unsigned t = blockIdx.x * kCol + threadIdx.x, tt = min(t, nxy - 1);
+  const unsigned t = blockIdx.x * (WHOLE ? kWhole : kCol) + threadIdx.x, tt = min(t, nxy - 1);
   const int i = (int)(tt % (unsigned)d.nx) + 1, j = (int)(tt / (unsigned)d.nx) + 1;
   double L = 0.0;
-  for (int k0 = 1, par = 0; k0 <= d.nz; k0 += kChunk, par ^= 1) {
-    level_sums(d, c0, d.p3(i, j, 0), k0, sum[par]);
-    if (threadIdx.y != 0) continue;
-    for (int k = k0; k < k0 + kChunk && k <= d.nz; ++k) L = L + sum[par][k - k0][threadIdx.x] * dz[k - 1] / 1.0e3;
+  if constexpr (WHOLE) {
+    whole_column(d, c0, d.p3(i, j, 0), dz, [&](int, double, double term) { L = L + term; });
+  } else {
+    __shared__ double term[2][kChunk][kCol];
+    for (int k0 = 1, par = 0; k0 <= d.nz; k0 += kChunk, par ^= 1) {
+      level_sums(d, c0, d.p3(i, j, 0), dz, k0, nullptr, term[par]);
+      if (threadIdx.y != 0) continue;
+      for (int k = k0; k < k0 + kChunk && k <= d.nz; ++k) L = L + term[par][k - k0][threadIdx.x];
+    }
   }
   if (threadIdx.y == 0 && t < nxy) out[t] = L;
 }
@@ -157,14 +215,21 @@ void put_i(std::string &o, int v, int w) {
 
 hipError_t launch_products(hipStream_t s, const ProdArgs &p) {
   const long long nxy = (long long)p.d.nx * p.d.ny;
-  hipLaunchKernelGGL(k_products, dim3((unsigned)((nxy + kCol - 1) / kCol)), dim3(kCol, kWaves), 0, s, p);
+  if (whole_columns(p.d))
+    hipLaunchKernelGGL((k_products<true>), dim3((unsigned)((nxy + kWhole - 1) / kWhole)), dim3(kWhole), 0, s, p);
+  else
+    hipLaunchKernelGGL((k_products<false>), dim3((unsigned)((nxy + kCol - 1) / kCol)), dim3(kCol, kWaves), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_column_load(hipStream_t s, const Dims &d, const double *c0, const double *dz, double *out) {
   const long long nxy = (long long)d.nx * d.ny;
-  hipLaunchKernelGGL(k_column_load, dim3((unsigned)((nxy + kCol - 1) / kCol)), dim3(kCol, kWaves), 0, s, d, c0, dz,
-                     out);
+  if (whole_columns(d))
+    hipLaunchKernelGGL((k_column_load<true>), dim3((unsigned)((nxy + kWhole - 1) / kWhole)), dim3(kWhole), 0, s, d, c0,
+                       dz, out);
+  else
+    hipLaunchKernelGGL((k_column_load<false>), dim3((unsigned)((nxy + kCol - 1) / kCol)), dim3(kCol, kWaves), 0, s, d,
+                       c0, dz, out);
   return hipGetLastError();
 }
 
