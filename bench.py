@@ -74,8 +74,9 @@ def effective_knobs(kind, st, tuning):
     if kind == "advect_x":
         return {"adv_x_rows": tuning["adv_x_rows"], "adv_fused": tuning["adv_fused"]}
     if kind in ("advect_y", "advect_z"):
-        return {"nb": tuning["nb_" + kind], "adv_groups": tuning["adv_groups_" + kind[-1]],
-                "adv_fused": tuning["adv_fused"]}
+        # register tiles, which take no setting of their own (no workload here
+        # is periodic without diffusion)
+        return {"adv_fused": tuning["adv_fused"]}
     d = kind[-1]
     n = {"x": st.nx, "y": st.ny, "z": st.nz}[d]
     nmax = tuning["part_max_line"] if d == "x" else tuning["part_max_line_strided"]

@@ -4,9 +4,11 @@ For each sweep kind it times the launch settings that do not change the
 results (bins one GPU thread carries along a line, bin groups per
 workgroup, row kernels, tile shapes of the partitioned line solves, the
 longest line those take) with the library's HIP-event kernel timers, on the
-live context.  The library's default is timed first and kept unless another
-setting is faster by more than `margin` (2 % by default), so that timing
-noise does not flip the choice.  The tuning steps advance the context's
+live context.  Settings that no kernel of the step reads are left alone (their
+times would differ by noise, and other sweeps, the adjoint's among them, read
+them too).  The library's default is timed first and kept unless another
+setting is faster by more than `margin` (2 % by default) in two measurements,
+so that timing noise does not flip the choice.  The tuning steps advance the context's
 state like ordinary steps; results of a step do not depend on the setting.
 Choices can be cached in a JSON file keyed by grid shape and bin count.
 """
@@ -35,6 +37,22 @@ PART_BINS = (0, 8, 4)
 PART_MAX_LINE = (512, 2048)
 # most Jacobi sweeps for strided lines beyond the partitioned solves (0: never)
 JACOBI_SWEEPS = 12
+
+
+def reached(st, param: str, use_diffusion: bool) -> bool:
+    """Whether a kernel of the whole-grid step reads the setting: the y and z
+    advection sweeps run in register tiles, which take none, except those of a
+    periodic step without diffusion (in place, streamed where the tiles do not
+    apply); the diffusion's settings belong to the theta-scheme's solves."""
+    if param in ("nb_advect_y", "adv_groups_y"):
+        return bool(st.is_periodic) and not use_diffusion and st.ny > 64
+    if param in ("nb_advect_z", "adv_groups_z"):
+        return bool(st.is_periodic) and not use_diffusion
+    if param == "adv_fused":
+        return use_diffusion  # the fused pass belongs to the step with diffusion
+    if param.startswith(("nb_diffuse", "x_tile", "part_", "jacobi")):
+        return use_diffusion and bool(st.use_cn)
+    return True
 
 
 def _key(st):
@@ -72,12 +90,8 @@ def autotune(T, use_diffusion: bool, steps: int = 2, candidates=(1, 2, 3, 4, 8),
             params.append(("jacobi_sweeps", ("diffuse_x", "diffuse_y", "diffuse_z")))
     for param, kind in params:
         kinds = kind if isinstance(kind, tuple) else (kind,)
-        if kinds[0].startswith("diffuse") and not use_diffusion:
+        if not reached(st, param, use_diffusion):
             continue
-        if param == "adv_fused" and not use_diffusion:
-            continue  # the fused pass belongs to the step with diffusion
-        if param in ("nb_advect_z", "adv_groups_z") and use_diffusion and T.tune_get("adv_fused"):
-            continue  # the vertical sweep runs inside the fused pass
         values = (X_TILES if param == "x_tile" else PART_BINS if param == "part_bins" else
                   (1, 0) if param == "adv_fused" else
                   (JACOBI_SWEEPS, 0) if param == "jacobi_sweeps" else
@@ -88,13 +102,10 @@ def autotune(T, use_diffusion: bool, steps: int = 2, candidates=(1, 2, 3, 4, 8),
                   (0, 1) if param.startswith("part_shape") else candidates)
         default = T.tune_get(param)
         values = (default,) + tuple(v for v in values if v != default)
-        times = {}
-        for nb in values:
-            if param.startswith("nb_") and nb > 1 and nb // 2 >= st.ns:
-                continue
-            if param.startswith("nb_diffuse") and nb == 3:
-                continue  # 3 bins per thread: the advection sweeps only
-            T.tune(**{param: nb})
+
+        def time_of(value):
+            nonlocal itime
+            T.tune(**{param: value})
             T.profile(True)
             for _ in range(steps):
                 itime += 1
@@ -104,11 +115,18 @@ def autotune(T, use_diffusion: bool, steps: int = 2, candidates=(1, 2, 3, 4, 8),
             T.profile(False)
             if param == "adv_fused":
                 # the whole advection of a step (the kinds it launches differ)
-                times[nb] = sum(prof[k][0] for k in kinds) / steps
-            else:
-                times[nb] = sum(prof[k][0] / max(prof[k][1], 1) for k in kinds)
+                return sum(prof[k][0] for k in kinds) / steps
+            return sum(prof[k][0] / max(prof[k][1], 1) for k in kinds)
+
+        times = {}
+        for nb in values:
+            if param.startswith("nb_") and nb > 1 and nb // 2 >= st.ns:
+                continue
+            if param.startswith("nb_diffuse") and nb == 3:
+                continue  # 3 bins per thread: the advection sweeps only
+            times[nb] = time_of(nb)
         best = min(times, key=times.get)
-        if times[best] > (1.0 - margin) * times[default]:
+        if times[best] > (1.0 - margin) * times[default] or time_of(best) > (1.0 - margin) * time_of(default):
             best = default
         T.tune(**{param: best})
         chosen[param] = (best, times)
