@@ -707,26 +707,21 @@ int jacobi_x_sweeps(ash3d_tr_ctx *x, const LineGeom &g, bool *all) {
   return sw == 0 ? 0 : std::min(sw, x->jacobi_sweeps);
 }
 
-// Cell offsets of the partitioned solves of direction dir: the state in
-// its own layout, the row factor cache in the sweep's (for x lines the
-// x<->y transposed one, a.d)
-PartLayout part_layout(const ash3d_tr_ctx *x, int dir, const DiffArgs &a) {
+// Cell offsets of the partitioned solves of direction dir (x lines take kappa,
+// sigma and K instead of the row factor cache, which lies along y)
+PartLayout part_layout(const ash3d_tr_ctx *x, int dir) {
   const Dims &o = x->d;
   PartLayout lay;
   lay.st0 = 1 + o.sy + o.sz;
   if (dir == 0) {
     lay.sta = o.sy; lay.stb = o.sz; lay.str = 1;
-    const Dims &t = a.d;  // transposed: cell (j, r, k) at (j+1) + t.sy*(r+1) + t.sz*(k+1)
-    lay.lr0 = 1 + t.sy + t.sz; lay.lra = 1; lay.lrb = t.sz; lay.lrr = t.sy;
     lay.sig = x->sx; lay.kk = x->kx;
     lay.ka = o.nx + 2; lay.kb = (long long)(o.nx + 2) * (o.ny + 2);
   } else {
     lay.sta = 1;
     lay.stb = (dir == 1) ? o.sz : o.sy;
     lay.str = (dir == 1) ? o.sy : o.sz;
-    lay.lr0 = lay.st0; lay.lra = lay.sta; lay.lrb = lay.stb; lay.lrr = lay.str;
   }
-  lay.lr_ncell = a.d.ncell;
   lay.kap = x->kap;
   return lay;
 }
@@ -746,7 +741,7 @@ int try_cn_partitioned(ash3d_tr_ctx *x, int dir, DiffArgs &a, int *rc, bool adjo
   if (dgtsv_sweep(x, dir, n)) return 0;
   const int hn = x->capturing && x->cap_dom[dir] ? 0 : host_ndom(x, dir);
   if (hn > 0) return 0;
-  const PartLayout lay = part_layout(x, dir, a);
+  const PartLayout lay = part_layout(x, dir);
   a.sel = 1;
   hipError_t e = launch_diff_cn_part(x->stream, a, lay, x->part_bins, x->part_shape[dir], adjoint);
   if (e != hipSuccess) *rc = fail(ASH3D_TR_EDEVICE, "partitioned line solve: %s", hipGetErrorString(e));
@@ -2463,7 +2458,7 @@ int ens_member_specs(ash3d_tr_ctx *x, int itime, double dt, double imp_fac, cons
     if (dir == 0) transpose_x_args(x, b, a);
     if ((rc = ensure_lr(x, dir, a)) || (rc = ensure_lu(x, dir, a, false))) return rc;
     a.sel = 1;
-    hipError_t e = spec_diff_cn_part(a, part_layout(x, dir, a), x->part_bins, x->part_shape[dir], &slots[q++]);
+    hipError_t e = spec_diff_cn_part(a, part_layout(x, dir), x->part_bins, x->part_shape[dir], &slots[q++]);
     if (e != hipSuccess) return fail(ASH3D_TR_EDEVICE, "ensemble diffusion dir %d: %s", dir, hipGetErrorString(e));
   }
   return q == kEnsSlots ? 0 : fail(ASH3D_TR_EINVAL, "ensemble step slots");

@@ -333,13 +333,11 @@ struct LineStats {
 // the row factors L, R of every cell of the sweep's lines (bin-independent)
 // and the LineStats of the active range
 hipError_t launch_line_rows(hipStream_t s, const DiffArgs &a, double *lr, const LineStats &st);
-// partitioned line solves (linesolve.hip): offsets of cell r of line (a, b)
-// are st0 + sta*a + stb*b + str*r in the state and lr0 + lra*a + lrb*b +
-// lrr*r in the row factor cache (R at + lr_ncell); hipErrorInvalidValue
-// when the active line length is outside [3, 512]
+// partitioned line solves (linesolve.hip): cell r of line (a, b) is at st0 +
+// sta*a + stb*b + str*r in the state and, y and z lines, in the row factor
+// cache; hipErrorInvalidValue when the active line length is outside [3, 2048]
 struct PartLayout {
   long long st0, sta, stb, str;
-  long long lr0, lra, lrb, lrr, lr_ncell;
   const double *kap = nullptr;  // cell volumes in the state's layout (x lines, adjoint)
   // x lines (str == 1), which form the row factors themselves: sigma_nx in
   // the state's layout and kx, cell i of line (a, b) at kk[ka*a + kb*b + i]

@@ -61,12 +61,11 @@ namespace ash3d {
 
 namespace {
 
-// Offsets of cell r of line (a, b): st0 + sta*a + stb*b + str*r in the
-// state (bin stride ncell) and lr0 + lra*a + lrb*b + lrr*r in the row
-// factor cache (L at lr[o], R at lr[o + lr_ncell]).
+// Offset of cell r of line (a, b): st0 + sta*a + stb*b + str*r in the state
+// (bin stride ncell) and, y and z lines, in the row factor cache (L there, R
+// ncell on).
 struct PartArgs {
   long long st0, sta, stb, str;
-  long long lr0, lra, lrb, lrr, lr_ncell;
   const double *kap;  // cell volumes at the state's cell offsets (x lines, adjoint)
   // x lines: sigma_nx likewise, and K of cell i of line (a, b) at kk[ka*a + kb*b + i]
   const double *sig, *kk;
@@ -162,7 +161,6 @@ __device__ __forceinline__ void cn_part_body(const DiffArgs &A, const PartArgs &
   const int wv = p / LP;     // part of the line (wave)
   const int a = a_first + ln;
   const bool has_line = owned(a);
-  const int ac = has_line ? a : g.Na;  // an existing line for masked lanes' reads
   const int rmin = g.rmin, rmax = g.rmax, n = rmax - rmin + 1, N = g.N;
   const bool line_on = has_line && a >= g.a0 && a <= g.a1 && b >= g.b0 && b <= g.b1;
   const int u0 = tg.group * Q.bins_wg;
@@ -296,13 +294,12 @@ __device__ __forceinline__ void cn_part_body(const DiffArgs &A, const PartArgs &
       stage([&](int m) { return dl[m] / kap_c[m]; }, Ls);
       stage([&](int m) { return dr[m] / kap_c[m]; }, Rs);
     } else {
-      const double *lr = A.lr + Q.lr0 + Q.lra * min(a_first + elem_l(0), g.Na) + Q.lrb * b;
       double l_[PF], r_[PF];
 #pragma unroll
       for (int m = 0; m < PF; ++m) {
-        const double *q = lr + Q.lrr * (long long)(rmin + row_of(m));
+        const double *q = A.lr + cell_of(m);
         l_[m] = q[0];
-        r_[m] = q[Q.lr_ncell];
+        r_[m] = q[ncell];
       }
       stage([&](int m) { return l_[m]; }, Ls);
       stage([&](int m) { return r_[m]; }, Rs);
@@ -808,7 +805,6 @@ static hipError_t diff_cn_part_any(hipStream_t s, const DiffArgs &a, const PartL
   const int n = a.g.rmax - a.g.rmin + 1;
   PartArgs q;
   q.st0 = lay.st0; q.sta = lay.sta; q.stb = lay.stb; q.str = lay.str;
-  q.lr0 = lay.lr0; q.lra = lay.lra; q.lrb = lay.lrb; q.lrr = lay.lrr; q.lr_ncell = lay.lr_ncell;
   q.kap = lay.kap;
   q.sig = lay.sig; q.kk = lay.kk; q.ka = lay.ka; q.kb = lay.kb;
   q.bins_wg = (bins_wg > 0 && bins_wg < a.d.ns) ? bins_wg : a.d.ns;
