@@ -33,6 +33,7 @@ struct TileArgs {
   AdvArgs A;
   int groups;   // bin groups (one wave each)
   int bins;     // bins per group
+  bool plain;   // the whole grid and every bin: nothing to look up per wave
 };
 
 // Ghost cells along the lines read as zero: Set_BC(1) zeroes them in y and
@@ -62,7 +63,7 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   const bool repeat = a0 + lane > g.Na;
   const int a = a0 + (int)al;
   const bool line_on = a >= g.a0 && a <= g.a1 && b >= g.b0 && b <= g.b1;
-  const bool plain = rmin == 1 && rmax == N && g.a0 == 1 && g.a1 == g.Na && g.b0 == 1 && g.b1 == g.Nb;
+  const bool plain = T.plain;
   const long long sL = line_stride(d, DIR), base = line_base(d, DIR, a0, b);
   auto row = [&](int r) { return base + sL * (long long)(r + 1); };  // uniform; + al
   double *junk = A.junk + lane + 64 * (int)(vb % (kJunk / 64));  // (of the wave with the line's last cells)
@@ -77,7 +78,7 @@ __device__ __forceinline__ void advect_tile_body(const TileArgs &T, const long l
   // line belongs to a tile with cells of the box).  The 3x3x3 box of a
   // 360x240x50x15 step without diffusion: 641 us, 1057 us with every tile
   // read.  Bit n - nlo of run: bin n is swept here
-  const unsigned group = (1u << (nhi - nlo)) - 1, on = A.aloft.bits(nlo, nhi);
+  const unsigned group = (1u << (nhi - nlo)) - 1, on = plain ? group : A.aloft.bits(nlo, nhi);
   const bool in_box = a0 <= g.a1 && a0 + 63 >= g.a0 && b >= g.b0 && b <= g.b1 && r0 <= rmax && r0 + M > rmin;
   const unsigned run = in_box ? on : 0u;
   for (unsigned z = group & ~run; z; z &= z - 1) {
@@ -290,7 +291,10 @@ hipError_t launch_tile(hipStream_t s, const AdvArgs &a, LaunchSpec *sp) {
   // that the last round of waves is short (15 bins in one group: 5 % slower
   // on 360x240x50)
   const long long want = std::max<long long>((2048 + tiles * S - 1) / (tiles * S), (a.d.ns + kTileBins - 1) / kTileBins);
-  TileArgs t{a, 1, a.d.ns};
+  TileArgs t{a, 1, a.d.ns, true};
+  for (int n = 0; n < a.d.ns; ++n) t.plain = t.plain && a.aloft.on(n);
+  const LineGeom &g = a.g;
+  t.plain = t.plain && g.rmin == 1 && g.rmax == g.N && g.a0 == 1 && g.a1 == g.Na && g.b0 == 1 && g.b1 == g.Nb;
   t.groups = (int)std::min<long long>(a.d.ns, want);
   t.bins = (a.d.ns + t.groups - 1) / t.groups;
   t.groups = (a.d.ns + t.bins - 1) / t.bins;
