@@ -15,7 +15,7 @@
 // on larger states, what bounds it (y at 240x160x50x8: 569 MB in 148 us, 3.9
 // TB/s).  Against one thread per line and 2 or 8 bins (k_diff_cn,
 // k_diff_cn_xrows, which keep the sweeps with row interchanges): 240x160x50x8
-// x, y, z 380, 347, 145 us -> 175, 148, 78 (z with the ts1 slot 118).
+// x, y, z 380, 347, 145 us -> 172, 146, 77 (z with the ts1 slot 118).
 // Quotients from inverses (fewer dependent operations) and two chunks in
 // flight gained nothing.  The arithmetic is dgtsv's, so the results are the
 // same bits.
@@ -302,7 +302,8 @@ hipError_t launch(hipStream_t s, const ExactArgs &e) {
 }  // namespace
 
 // Four waves per workgroup share the row coefficients (two or one for fewer
-// bins), eight rows per chunk.  240x160x50x8 x, y, z: 161, 138, 110 us; two
+// bins), eight rows per chunk.  Measured when every line's right-hand sides
+// still went through the ts1 slot, 240x160x50x8 x, y, z: 161, 138, 110 us; two
 // waves 178, 133, 134; eight 240, 143, 121 (too few workgroups for the
 // serial chains of one to fill the others' waits); 16 rows 152, 136, 117 but
 // 254 against 238 on 241-cell rows, at 250 more registers.

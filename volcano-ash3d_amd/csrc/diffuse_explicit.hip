@@ -11,7 +11,7 @@
 // at their borders are copied to the ts1 slot beforehand and read from there.
 // The ghost cells along the lines are not read: they hold the edge cells
 // (periodic x: the wrapped ones, :317-327).  Bound by HBM latency and
-// bandwidth; 181x133x41x7 (6.9 M bin-cells): x, y, z 25, 41 (borders included), 29 us against
+// bandwidth; 181x133x41x7 (6.9 M bin-cells): x, y, z 25, 40 (borders included), 27 us against
 // 254 (with the transposes of the state that the x lines went through), 147
 // and 58 us for one thread per line.
 // The arithmetic is the reference's, expression by expression.

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kRed) void k_dt_partials(DtArgs A) {
 // wave a row at a time in blocks of kSlabCols columns, all loads of a row
 // in flight: the column maxima stay in registers, a row costs one wave
 // reduction, and an atomic is issued only for a value above the stored one
-// (175 MB of 241x161x45x10 in 45 us against 113 us with a reduction per 64
+// (140 MB of 241x161x45x10 in 50 us against 113 us with a reduction per 64
 // cells and an atomic per column and plane).
 constexpr int kSlabChunks = 6, kSlabCols = 64 * kSlabChunks, kSlabRows = 64;
 

@@ -31,7 +31,7 @@ constexpr double M_2_MM = 1.0e3;     // :281
 // over the bins in the reference's order with eight bins' loads in flight,
 // into LDS; then the first wave folds the chunk's levels upward.  One pass
 // over the state, bound by HBM bandwidth: 518 MB of a 360x240x50x15 state in
-// 125 us (products) and 120 us (column load), against 349 and 338 us with
+// 112 us (products) and 100 us (column load), against 347 and 338 us with
 // one thread per column, which kept a load or two in flight per lane.
 constexpr int kCol = 64, kWaves = 8, kChunk = 16;
 

@@ -10,7 +10,7 @@
 // each over a fixed set of cells in a fixed order, then a fixed-order sum
 // of the partials.  The aloft sum reads the state once, a wave per x row
 // (lanes along x, so that a row needs one division for its indices instead
-// of several per cell): 518 MB of a 360x240x50x15 state in 125 us against
+// of several per cell): 518 MB of a 360x240x50x15 state in 108 us against
 // 210 us with one thread per strided cell.
 #include "common.hpp"
 
