@@ -348,11 +348,13 @@ int set_bc1(ash3d_tr_ctx *x, bool velocities, double *state = nullptr, bool conc
   ProfScope ps(x, ASH3D_PROF_BC);
   // Set_BC(1) on velocities is a projection (every ghost a copy of an
   // interior or wrapped cell that the pass does not write), so it is
-  // skipped while the ghosts already hold its values (a captured step runs
-  // it before the capture, and before a replay when velocities changed)
-  if (velocities && !x->vel_bc_ok)
-    HIPCHK(launch_set_bc1_vel(x->stream, x->d, x->periodic, x->vx, x->vy, x->vz, x->vf));
-  if (velocities) x->vel_bc_ok = true;
+  // skipped while the ghosts already hold its values (a captured step leaves
+  // it to the replay, which runs it first when velocities changed)
+  if (velocities && !x->capturing) {
+    if (!x->vel_bc_ok)
+      HIPCHK(launch_set_bc1_vel(x->stream, x->d, x->periodic, x->vx, x->vy, x->vz, x->vf));
+    x->vel_bc_ok = true;
+  }
   if (conc) HIPCHK(launch_set_bc1_conc(x->stream, x->d, x->periodic, state ? state : x->ts0()));
   return 0;
 }
@@ -2051,9 +2053,8 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
   for (int k = 0; k < 3; ++k) x->cap_dom[k] = false;
   x->graph_dtv[slot] = -1.0;
   if (use_diffusion && x->adv_fused && (rc = ensure_dtv(x, dt))) return rc;  // (outside the capture)
-  // (outside the capture too) the velocity ghosts, the line factors, and
-  // which sweeps need no dgtsv-order alternative
-  if ((rc = set_bc1(x, true, nullptr, false))) return rc;
+  // (outside the capture too) the line factors, and which sweeps need no
+  // dgtsv-order alternative
   if (use_diffusion && use_cn) {
     int32_t b[6];
     full_bounds(x, b);
