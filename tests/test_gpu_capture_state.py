@@ -42,3 +42,25 @@ def test_captures_leave_velocity_ghosts(pkg, tr, use_diffusion, periodic):  # no
         assert np.array_equal(getattr(a, n), getattr(b, n)), n
     E.close()
     G.close()
+
+
+def test_captures_follow_an_eager_diffusion(pkg, tr):  # noqa: F811
+    """Explicit diffusion: refused before an x sweep on the present geometry
+    and diffusivities, as a theta-scheme step's capture is."""
+    st = pkg.workloads.random_state(14, 9, 7, 2, seed=2, latlon=True, use_cn=False)
+    st.dt *= 0.2
+    with tr.Transport(st) as T:
+        T.transport_step(1, False)
+        with pytest.raises(tr.Ash3dError, match="capture after an eager step"):
+            T.graph_capture(2, True)
+        T.graph_capture(2, False)
+        T.diff_x()
+        T.graph_capture(2, True)
+        T.sync_from_host(tr.SYNC_DIFFK)
+        with pytest.raises(tr.Ash3dError, match="capture after an eager step"):
+            T.graph_capture(2, True)
+        T.step_glue()
+        T.transport_step(3, True)
+        T.graph_capture(2, True)
+        T.graph_launch(2)
+        T.synchronize()

@@ -193,6 +193,9 @@ struct ash3d_tr_ctx {
   // transposed kappa, sigma_nx and kx (rebuilt after a geometry/K upload)
   double *tq = nullptr, *tkap = nullptr, *tsx = nullptr, *tkx = nullptr;
   bool tgeom_valid = false;
+  // an explicit x sweep has run on the present geometry and K (captured steps
+  // with explicit diffusion follow one)
+  bool xexp_ok = false;
   // adjoint: lambda, snapshots of the recomputed sweep inputs, line-solve
   // scratch, an outflow sink for recomputed sweeps, source-gradient slots
   double *lam = nullptr, *snap_b = nullptr, *snap_z = nullptr, *adj_sb = nullptr, *sink = nullptr;
@@ -862,6 +865,7 @@ int sweep_diffuse(ash3d_tr_ctx *x, int dir, int use_cn, double dt, double imp_fa
   } else {
     ProfScope ps(x, ASH3D_PROF_DIFFUSE_X + dir);
     HIPCHK(launch_diff_explicit(x->stream, a, x->periodic));
+    if (dir == 0) x->xexp_ok = true;
   }
   x->ts1_state = TS1_MIRROR;
   return 0;
@@ -1147,7 +1151,7 @@ int ash3d_tr_sync_from_host(ash3d_tr_ctx *x, uint32_t mask) {
     if ((rc = upload(x, x->vf, h.vf_pd, x->n_conc(), 0.0))) return rc;
   if (mask & ASH3D_SYNC_GEOMETRY) x->dtv_ok = false;
   if (mask & (ASH3D_SYNC_GEOMETRY | ASH3D_SYNC_DIFFK)) {
-    x->tgeom_valid = false;
+    x->tgeom_valid = x->xexp_ok = false;
     x->lr_ok[0] = x->lr_ok[1] = x->lr_ok[2] = false;
   }
   if (mask & ASH3D_SYNC_GEOMETRY) {
@@ -2041,8 +2045,9 @@ int ash3d_tr_graph_capture(ash3d_tr_ctx *x, int32_t itime, double dt, int32_t us
   if (x->prof_on) return fail(ASH3D_TR_EINVAL, "kernel timing is on; switch it off before capturing");
   if (use_diffusion && use_cn && !(x->lu[0] && x->lu[1] && x->lu[2] && x->junk))
     return fail(ASH3D_TR_EINVAL, "capture after an eager step (line-solve factors not allocated)");
-  if (use_diffusion && use_cn && !x->tgeom_valid)
-    return fail(ASH3D_TR_EINVAL, "capture after an eager step (transposed geometry not built)");
+  if (use_diffusion && !x->tgeom_valid && (use_cn || !x->xexp_ok))
+    return fail(ASH3D_TR_EINVAL, "capture after an eager step (%s)",
+                use_cn ? "transposed geometry not built" : "no diffusion along x on this geometry and K yet");
   HIPCHK(hipStreamSynchronize(x->stream));
   const int slot = itime % 2;
   for (hipGraphExec_t *g : {&x->graph[slot], &x->graph_any[slot]})
