@@ -64,3 +64,37 @@ def test_captures_follow_an_eager_diffusion(pkg, tr):  # noqa: F811
         T.graph_capture(2, True)
         T.graph_launch(2)
         T.synchronize()
+
+
+@pytest.mark.parametrize("change", ["box", "dt"])
+def test_captures_leave_later_sweeps_right(pkg, oracle, tr, change):  # noqa: F811
+    """A capture whose line factors are not the cached ones (another box or
+    time step came before) forms them at once: eager sweeps after it, and
+    replays of either parity first, are bitwise the oracle's."""
+    st = pkg.workloads.random_state(18, 7, 16, 2, seed=8, latlon=True)
+    st.concen_pd[..., 1] = st.concen_pd[..., 0]
+    a, b = st.copy(), st.copy()
+    O, T = oracle.Oracle(a), tr.Transport(b)
+    T.tune(line_solver="exact")
+    for S, h in ((O, a), (T, b)):
+        S.transport_step(1, True)
+        if change == "box":
+            h.bounds = (3, 9, 2, 5, 4, 11)
+            for name in ("diffCN_x", "diffCN_y", "diffCN_z"):
+                getattr(S, name)()
+            h.bounds = (1, 18, 1, 7, 1, 16)
+        else:
+            h.dt *= 0.7
+    T.graph_capture(2, True)
+    T.graph_capture(3, True)
+    for S in (O, T):
+        S.DiffuseVert()
+        S.DiffuseHorz(1)
+    for itime in (3, 2):
+        O.step_glue()
+        O.transport_step(itime, True)
+        T.graph_launch(itime)
+    T.sync_to_host()
+    for n in ("concen_pd", "outflow_yz1_pd", "outflow_xz2_pd", "outflow_xy1_pd"):
+        assert np.array_equal(getattr(a, n), getattr(b, n)), n
+    T.close()
